@@ -23,6 +23,7 @@ HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
 COMMON = [
     f"--offload-arch={ARCH}", "-O3", "-std=c++17", "-fPIC",
     "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops",
+    "-fconstexpr-steps=100000000",     # the FFT root tables (csrc/bm_twiddle.h)
     "-Wno-unused-result", "-I", str(PKG.parent / "include"),
 ]
 SOURCES = ["bm_demag.hip", "bm_mlayer.hip", "bm_batch.hip", "bm_adjoint.hip", "bm_row_rkdp.hip", "bm_row_rk4.hip", "bm_row_heun.hip", "bm_ode.hip", "bm_common.cpp", "bm_tensor.cpp", "bm_ovf2.cpp"]

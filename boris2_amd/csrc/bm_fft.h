@@ -11,12 +11,13 @@
 // the first N/2 outputs are needed, callers store only e < E/2 and the dead outputs of the
 // last butterfly are eliminated.
 //
-// Twiddles come from FP64 sincospi (rounded to the working precision), computed once per
-// thread per kernel (they depend only on the thread's butterfly indices) and kept in
-// registers across every line the thread transforms.
+// FP32 twiddles are read from constant tables (bm_twiddle.h), FP64 ones (kernel set-up only)
+// come from sincospi; both once per thread per kernel (they depend only on the thread's
+// butterfly indices), kept in registers across every line the thread transforms.
 #pragma once
 
 #include <hip/hip_runtime.h>
+#include "bm_twiddle.h"
 
 namespace bm {
 
@@ -218,9 +219,15 @@ template <int N, typename T> struct Twiddles {
 				int j = t + b * TT, k = j % Ns;
 #pragma unroll
 				for (int r = 1; r < R; r++) {
-					double sn, cs;
-					sincospi(-2.0 * (double)(k * r) / (double)(Ns * R), &sn, &cs);
-					w[off + b * (R - 1) + r - 1] = mk((T)cs, (T)sn);
+					if constexpr (sizeof(T) == 4) {
+						const float2 q = tw_roots<Ns * R>()[k * r];
+						w[off + b * (R - 1) + r - 1] = mk((T)q.x, (T)q.y);
+					}
+					else {
+						double sn, cs;
+						sincospi(-2.0 * (double)(k * r) / (double)(Ns * R), &sn, &cs);
+						w[off + b * (R - 1) + r - 1] = mk((T)cs, (T)sn);
+					}
 				}
 			}
 			init_stage<s + 1>(t);

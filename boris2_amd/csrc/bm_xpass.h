@@ -51,7 +51,7 @@ template <int HX> struct XThread {
 		t = threadIdx.x % T; rl = threadIdx.x / T;
 		tw.init(t);
 #pragma unroll
-		for (int e = 0; e < E; e++) { double s, c; sincospi(-(double)(t + T * e) / HX, &s, &c); wk[e] = mk((float)c, (float)s); }
+		for (int e = 0; e < E; e++) { const float2 q = tw_roots<2 * HX>()[t + T * e]; wk[e] = mk(q.x, q.y); }
 	}
 };
 
