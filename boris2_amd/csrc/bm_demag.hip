@@ -673,6 +673,7 @@ int launch_fwd_x(int HX, bool full, const float* M, float2* Sx, int ny, int nz, 
 	if (gen && (full || adv)) return fail(BM_ERR_STATE, "general row length: no periodic x, no fused advance");
 	const int f = (full || gen) ? 1 : xtile_factor(true);
 	FwdArgs a{ M, Sx, ny, nz, ntl, 0, E0, sM1, Mout, dT5, gen ? nx : HX, zoff, nzl };
+	if (f == 1 && xs_few_rows(HX, ny, nz, ncu)) return launch_fwd_xs(HX, full, a, st);
 	switch (HX) {
 #define C_(V_) case V_: { constexpr int TY1 = XTile<V_>::v; int TY = TY1 * f; a.ntiles = (ny + TY - 1) / TY; dim3 g(grid_for(nz * a.ntiles, ncu, 2)); \
 		const FwdArgs* nb = nullptr; \
@@ -706,6 +707,7 @@ int launch_inv_x(int HX, bool full, int mode, const float2* Sx, float* out, int 
 {
 	const bool gen = !full && nx && nx != HX;
 	const int f = (mode == 0 && !full && !gen) ? xtile_factor(false) : 1;
+	if (f == 1 && xs_few_rows(HX, ny, nz, ncu)) return launch_inv_xs(HX, full, mode, Sx, out, ny, nz, ntl, scale, st, M, epart, gen ? nx : HX, zoff, nzl);
 	switch (HX) {
 #define C_(V_) case V_: { constexpr int TY1 = XTile<V_>::v; int TY = TY1 * f, nt = (ny + TY - 1) / TY; dim3 g(grid_for(3 * nz * nt, ncu, 2)); \
 		const PassBatch* nb = nullptr; \
@@ -719,8 +721,10 @@ int launch_inv_x(int HX, bool full, int mode, const float2* Sx, float* out, int 
 	return fail(BM_ERR_SIZE, "no x plan");
 }
 
-int inv_x_nwork(int HX, int ny, int nz)
+// energy partials of the inverse x pass: one per work item of the variant that runs
+int inv_x_nwork(int HX, int ny, int nz, int ncu)
 {
+	if (xs_few_rows(HX, ny, nz, ncu)) return xs_parts(HX, ny, nz);
 	switch (HX) {
 #define C_(V_) case V_: { int TY = XTile<V_>::v; return 3 * nz * ((ny + TY - 1) / TY); }
 	BM_FOR_X_SIZES(C_)
@@ -1291,7 +1295,7 @@ static int demag_create(int nx, int ny, int nz, double hx, double hy, double hz,
 	const size_t sxbytes = (size_t)3 * nz * d->ntl * d->NC * kLT * sizeof(float2);
 	const size_t sbytes = d->is2d ? 0 : (size_t)3 * nz * d->NC * d->Sp * sizeof(float2);
 	d->kcount = d->is2d ? 4LL * d->NC * d->NYH : 6LL * d->NZH * d->NC * d->NYH;
-	d->ecap = std::max(1, inv_x_nwork(d->Nx / 2, ny, nz));
+	d->ecap = std::max(1, inv_x_nwork(d->Nx / 2, ny, nz, d->ncu));
 	if (hipMalloc(&d->Sx, sxbytes) != hipSuccess || (sbytes && hipMalloc(&d->S, sbytes) != hipSuccess)
 		|| hipMalloc(&d->K, d->kcount * sizeof(float)) != hipSuccess || hipMalloc(&d->ebuf, (size_t)d->ecap * sizeof(double)) != hipSuccess) {
 		bm_demag_destroy(d);
@@ -1352,7 +1356,7 @@ extern "C" int bm_demag_convolute(bm_demag_t d, const float* M, float* Heff, int
 	if (rc) return rc;
 	const float scale = (float)(1.0 / ((double)d->Nx * d->Ny * d->Nz));
 	if (energy) {
-		const int np = inv_x_nwork(HX, d->ny, d->nz);
+		const int np = inv_x_nwork(HX, d->ny, d->nz, d->ncu);
 		if (np > d->ecap) return fail(BM_ERR_STATE, "energy partial buffer too small");
 		prof_mark_begin(PK_INV_X, st);
 		rc = launch_inv_x(HX, d->full[0], clear_out ? 1 : 2, d->Sx, Heff, d->ny, d->nz, d->ntl, scale, d->ncu, st, M, d->ebuf, d->nx);
@@ -1515,7 +1519,7 @@ int bm::pass_fwd_x_plane(int nx, const float* M, float2* Sx, int ny, int plane, 
 	return rc;
 }
 
-int bm::x_plane_parts(int nx, int ny) { return std::max(1, inv_x_nwork(nx, ny, 1)); }
+int bm::x_plane_parts(int nx, int ny) { return std::max(1, inv_x_nwork(nx, ny, 1, device_cu_count())); }
 
 int bm::pass_inv_x_plane(int nx, int mode, const float2* Sx, float* out, int ny, int plane, int nzl, int ntl, float scale, int ncu,
 	hipStream_t st, const float* M, double* epart, float* energy, bool full)
@@ -1525,7 +1529,7 @@ int bm::pass_inv_x_plane(int nx, int mode, const float2* Sx, float* out, int ny,
 	int rc = launch_inv_x(nx, full, mode, Sx, out, ny, 1, ntl, scale, ncu, st, energy ? M : nullptr, energy ? epart : nullptr, 0, plane, nzl);
 	prof_mark_end(PK_INV_X, st);
 	if (rc || !energy) return rc;
-	hipLaunchKernelGGL(k_energy_final, dim3(1), dim3(kBlock), 0, st, epart, inv_x_nwork(nx, ny, 1), (size_t)(full ? 2 * nx : nx) * ny, energy);
+	hipLaunchKernelGGL(k_energy_final, dim3(1), dim3(kBlock), 0, st, epart, inv_x_nwork(nx, ny, 1, ncu), (size_t)(full ? 2 * nx : nx) * ny, energy);
 	return BM_OK;
 }
 
@@ -1559,6 +1563,12 @@ int bm::batch_fwd_x(int nx, bool full, LaunchShape sh, const FwdArgs* h_tab, con
 {
 	int mx = 1;
 	for (int b = 0; b < nb; b++) mx = std::max(mx, h_tab[b].nz * h_tab[b].ntiles);
+	if (!sh.f) {
+		// default: the few-rows form while all meshes together have few
+		int rows = 0;
+		for (int b = 0; b < nb; b++) rows += h_tab[b].ny * h_tab[b].nz;
+		if (xs_few_rows(nx, rows, 1, ncu)) return batch_fwd_xs(nx, full, h_tab, d_tab, nb, st);
+	}
 	const int f = full ? 1 : sh.f ? sh.f : xtile_factor(true);
 	const dim3 g(grid_for(mx, ncu, sh.per_cu ? sh.per_cu : 2), nb);
 	FwdArgs a{};
@@ -1579,6 +1589,11 @@ int bm::batch_inv_x_planar(int nx, bool full, LaunchShape sh, const PassBatch* h
 {
 	int mx = 1;
 	for (int b = 0; b < nb; b++) mx = std::max(mx, 3 * h_tab[b].nz * h_tab[b].ntiles);
+	if (!sh.f) {
+		int rows = 0;
+		for (int b = 0; b < nb; b++) rows += h_tab[b].ny * h_tab[b].nz;
+		if (xs_few_rows(nx, rows, 1, ncu)) return batch_inv_xs_planar(nx, full, h_tab, d_tab, nb, st);
+	}
 	const int f = full ? 1 : sh.f ? sh.f : xtile_factor(false);
 	const dim3 g(grid_for(mx, ncu, sh.per_cu ? sh.per_cu : 2), nb);
 	switch (nx) {

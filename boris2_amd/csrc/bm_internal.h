@@ -110,6 +110,16 @@ struct FwdArgs {
 	// whose layout has nzl planes per component (0, 0: the planes of M, nz per component)
 	int zoff, nzl;
 };
+// The x passes with one component per wave group (bm_xsplit.h): whether a launch over nz planes
+// of ny rows takes them (row: the fused row kernel), their energy partials, and their launchers
+// (arguments as the plain x passes'; nx: cells per row, HX unless the row is of the general length).
+bool xs_few_rows(int HX, int ny, int nz, int ncu, bool row = false);
+int xs_parts(int HX, int ny, int nz);
+int launch_fwd_xs(int HX, bool full, const FwdArgs& a, hipStream_t st);
+int launch_inv_xs(int HX, bool full, int mode, const float2* Sx, float* out, int ny, int nz, int ntl, float scale, hipStream_t st,
+	const float* M, double* epart, int nx, int zoff, int nzl);
+int batch_fwd_xs(int HX, bool full, const FwdArgs* h_tab, const FwdArgs* d_tab, int nb, hipStream_t st);
+int batch_inv_xs_planar(int HX, bool full, const struct PassBatch* h_tab, const struct PassBatch* d_tab, int nb, hipStream_t st);
 // Per-mesh arguments of the other passes in a batched launch (the fields each pass uses;
 // the y passes take ny as the data rows of a line).
 struct PassBatch {

@@ -19,6 +19,7 @@
 #include "bm_internal.h"
 #include "bm_stage.h"
 #include "bm_xpass.h"
+#include "bm_xsplit.h"
 
 namespace bm {
 
@@ -235,9 +236,17 @@ int launch_row_t(const bm_demag_s* d, const StageArgs& a, float scale, hipStream
 		return BM_OK;
 	}
 	switch (d->nx) {
-#define C_(V_) case V_: { constexpr int TY = XTile<V_>::v; const int nt = (d->ny + TY - 1) / TY; \
+#define C_(V_) case V_: { \
+	if constexpr (xs_ok<V_>()) if (xs_few_rows(V_, d->ny, d->nz, d->ncu, true)) { \
+		const int ns = (d->ny + XSplit<V_>::RP - 1) / XSplit<V_>::RP, g = d->nz * ns; \
+		hipLaunchKernelGGL((k_rows<V_, METHOD, STEP, R2C>), dim3((g + 7) / 8 * 8), dim3(XSplit<V_>::BS), 0, st, a, d->Sx, d->ntl, ns, scale); \
+		return BM_OK; \
+	} \
+	if constexpr (!xs_row_only<V_>()) { \
+		constexpr int TY = XTile<V_>::v; const int nt = (d->ny + TY - 1) / TY; \
 		hipLaunchKernelGGL((k_row<V_, TY, METHOD, STEP, R2C>), dim3(row_grid(d->nz * nt, d->ncu)), dim3(kXBlock), 0, st, a, d->Sx, d->ntl, nt, scale); \
-		return BM_OK; }
+		return BM_OK; \
+	} } break;
 	BM_FOR_ROW_SIZES(C_)
 #undef C_
 	}

@@ -46,9 +46,10 @@ template <int HX> struct XThread {
 	Twiddles<HX, float> tw;
 	C2<float> wk[E];   // W^k = exp(-i pi k / HX), k = t + T e
 
-	__device__ __forceinline__ void init()
+	__device__ __forceinline__ void init() { rl = threadIdx.x / T; init_at(threadIdx.x % T); }
+	__device__ __forceinline__ void init_at(int lane)
 	{
-		t = threadIdx.x % T; rl = threadIdx.x / T;
+		t = lane;
 		tw.init(t);
 #pragma unroll
 		for (int e = 0; e < E; e++) { const float2 q = tw_roots<2 * HX>()[t + T * e]; wk[e] = mk(q.x, q.y); }

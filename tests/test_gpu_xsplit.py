@@ -1,0 +1,76 @@
+"""The x passes and the row kernel with one component per wave group (few rows): every row length
+that takes them, at rows fewer than, equal to and one more than a workgroup's, against the FP64
+oracle.  Bars: the field's parity bar of 1e-6 relative L2, one step's 1e-6 of M (FP32 rounding of a
+few operations on values of one size, a step changes M by less than a tenth)."""
+import numpy as np
+import pytest
+import torch
+
+from boris2_amd import api
+import oracle_lib as O
+
+pytestmark = pytest.mark.gpu
+H = (4e-9, 4e-9, 4e-9)
+ALL = api.BM_MOD_DEMAG | api.BM_MOD_EXCHANGE | api.BM_MOD_ANIS_UNI | api.BM_MOD_ZEEMAN
+
+
+def nz_open(nz):
+    N = 1
+    while nz > 1 and N < 2 * nz:
+        N *= 2
+    return N
+
+
+def rel(a, b):
+    return np.linalg.norm(a - b) / np.linalg.norm(b)
+
+
+@pytest.mark.parametrize("n", [(2, 65, 1), (4, 33, 2), (6, 64, 1), (8, 31, 2), (12, 65, 1), (16, 33, 2), (24, 31, 1), (32, 17, 2),
+                               (48, 15, 1), (64, 9, 3), (96, 8, 1), (128, 5, 2), (192, 3, 2), (256, 3, 3), (384, 1, 2), (512, 5, 1),
+                               (768, 3, 1), (1024, 2, 2), (33, 10, 2), (100, 7, 1)])
+def test_field_set_added_planar_and_energy(gpu, n):
+    nc = n[0] * n[1] * n[2]
+    M0 = api.random_magnetisation(nc, 8e5, 11).astype(np.float32)
+    M = torch.from_numpy(M0).cuda()
+    d = api.Demag(n, H)
+    ref = O.OracleDemag(n, H, Nz_override=nz_open(n[2]))(M0.astype(np.float64))
+    e = torch.zeros(1, device="cuda")
+    Hs = d.convolute(M, energy=e)
+    base = torch.full_like(M, 1e4)
+    Ha = d.convolute(M, base.clone(), clear_out=False)
+    assert rel(Hs.cpu().numpy().astype(np.float64), ref) <= 1e-6
+    assert rel(Ha.cpu().numpy().astype(np.float64) - 1e4, ref) <= 1e-6
+    assert rel(d.convolute_planar(M).cpu().numpy().T.astype(np.float64), ref) <= 1e-6
+    want = -api.MU0 / 2 * (M0.astype(np.float64) * ref).sum() / nc
+    assert abs(e.item() - want) <= 1e-6 * api.MU0 / 2 * 8e5 * np.linalg.norm(ref) / np.sqrt(nc)
+    d.close()
+
+
+@pytest.mark.parametrize("n", [(64, 9, 1), (128, 5, 2), (192, 3, 1), (256, 3, 2), (384, 2, 2), (512, 5, 1), (768, 3, 1), (1024, 3, 1), (8, 65, 2)])
+@pytest.mark.parametrize("method", [api.BM_EVAL_RK4, api.BM_EVAL_RKDP54, api.BM_EVAL_TEULER, api.BM_EVAL_AHEUN])
+def test_steps(gpu, n, method):
+    nc = n[0] * n[1] * n[2]
+    p = api.FMParams(Ms=1e6, A=1.5e-11, alpha=0.1, K1=5e5, ea=(0.0, 0.0, 1.0), Ha=(0.0, 0.0, 4e4), modules=ALL)
+    M0 = api.random_magnetisation(nc, p.Ms, 5).astype(np.float32)
+    s = api.FMSolver(method, n, H, p, M0)
+    dt = 2e-15 if method == api.BM_EVAL_AHEUN else 1e-14       # no rejected step; the largest step, so no other one
+    s.set_dt(dt)
+    s.set_astep(dT_max=dt)
+    s.run_to_iteration(2)
+    o = O.OracleSim(method, n, H, p)
+    o.set_M(M0.astype(np.float64))
+    o.set_dt(dt)
+    o.set_astep(dtmax=dt)
+    o.run_to_iteration(2)
+    assert rel(s.M.cpu().numpy().astype(np.float64), o.get_M()) <= 1e-6
+    s.close()
+
+
+@pytest.mark.parametrize("n,pbc", [((64, 9, 2), (3, 0, 0)), ((256, 6, 1), (2, 2, 0)), ((512, 4, 2), (2, 0, 0)), ((48, 16, 1), (2, 1, 0))])
+def test_periodic_rows(gpu, n, pbc):
+    nc = n[0] * n[1] * n[2]
+    M0 = api.random_magnetisation(nc, 8e5, 3).astype(np.float32)
+    d = api.Demag(n, H, pbc)
+    ref = O.OracleDemag(n, H, pbc=pbc)(M0.astype(np.float64))
+    assert rel(d.convolute(torch.from_numpy(M0).cuda()).cpu().numpy().astype(np.float64), ref) <= 1e-6
+    d.close()
