@@ -97,6 +97,11 @@ struct bm_batch_s {
 	std::vector<Tab<PassBatch>> inv, ty, tz, ty2;
 	std::vector<Tab<MlBatch>> tml;
 	std::vector<Tab<PassBatch>> tyz[2];
+	// meshes whose middle passes run as the column pass (bm_col.hip), by N.y, kind and periodic y:
+	// those it serves whose y, z, 2D y, fused and product groups all have their default shapes
+	struct ColGroup { int Ny, kind; bool full; Tab<ColBatch> t; };
+	std::vector<ColGroup> gcol;
+	bool no_col = false;                   // while the autotuner times the separate passes
 	Tab<StageArgs> stage[2];               // [input parity]
 	Tab<int> choff;                        // first flat chunk of kBS cells of each mesh (nb + 1)
 	void* dev_tables = nullptr;
@@ -319,6 +324,33 @@ int build_tables(bm_batch_s* o)
 {
 	const int nb = o->nb;
 	if (o->dev_tables) { (void)hipFree(o->dev_tables); o->dev_tables = nullptr; }
+	std::vector<char> col((size_t)nb, 0);
+	o->gcol.clear();
+	{
+		std::vector<char> pinned((size_t)nb, 0);
+		for (const std::vector<Group>* gs : { &o->gy, &o->gz, &o->gy2, &o->gml, &o->gyz[0], &o->gyz[1] })
+			for (const Group& G : *gs)
+				for (int q = 0; q < 2; q++) if (G.sh[q].f || G.sh[q].per_cu || G.sh[q].radix) for (int b : G.meshes) pinned[(size_t)b] = 1;
+		for (int b = 0; b < nb; b++) {
+			if (o->no_col || pinned[(size_t)b] || (!o->ml[b] && !o->dm[b])) continue;
+			int Ny, kind; bool full = false; ColBatch t;
+			if (o->ml[b]) {
+				const MlView v = mlayer_view(o->ml[b]);
+				if (!col_ok(v.Ny, 0, v.L, v.NC, o->ncu)) continue;
+				Ny = v.Ny; kind = 0; t = ColBatch{ v.Sx, v.K, v.L, v.NC, v.NYH, v.ntl, v.ny };
+			}
+			else {
+				const bm_demag_s* d = o->dm[b];
+				if (!demag_col(d)) continue;
+				Ny = d->Ny; kind = d->Nz; full = d->full[1]; t = ColBatch{ d->Sx, d->K, d->nz, d->NC, d->NYH, d->ntl, full ? d->Ny : d->ny };
+			}
+			col[(size_t)b] = 1;
+			bm_batch_s::ColGroup* g = nullptr;
+			for (auto& q : o->gcol) if (q.Ny == Ny && q.kind == kind && q.full == full) g = &q;
+			if (!g) { o->gcol.push_back({ Ny, kind, full, {} }); g = &o->gcol.back(); }
+			g->t.h.push_back(t);
+		}
+	}
 	for (int par = 0; par < 2; par++) o->fwd[par].assign(o->gx.size(), Tab<FwdArgs>());
 	o->inv.assign(o->gx.size(), Tab<PassBatch>());
 	o->ty.assign(o->gy.size(), Tab<PassBatch>());
@@ -329,6 +361,7 @@ int build_tables(bm_batch_s* o)
 		o->tyz[q].assign(o->gyz[q].size(), Tab<PassBatch>());
 		for (size_t g = 0; g < o->gyz[q].size(); g++)
 			for (int b : o->gyz[q][g].meshes) {
+				if (col[(size_t)b]) continue;
 				bm_demag_s* d = o->dm[b];
 				PassBatch pb{}; pb.Sx = d->Sx; pb.K = d->K; pb.nz = d->nz; pb.NC = d->NC; pb.NYH = d->NYH; pb.ntl = d->ntl; pb.ny = d->ny;
 				o->tyz[q][g].h.push_back(pb);
@@ -358,6 +391,7 @@ int build_tables(bm_batch_s* o)
 	}
 	for (size_t g = 0; g < o->gy.size(); g++)
 		for (int b : o->gy[g].meshes) {
+			if (col[(size_t)b]) continue;
 			PassBatch q{};
 			if (o->ml[b]) { const MlView v = mlayer_view(o->ml[b]); q.S = v.S; q.Sx = v.Sx; q.Sp = v.Sp; q.NC = v.NC; q.ntl = v.ntl; q.nlines = 3 * v.L * v.NC; q.ny = v.ny; }
 			else { bm_demag_s* d = o->dm[b]; q.S = d->S; q.Sx = d->Sx; q.Sp = d->Sp; q.NC = d->NC; q.ntl = d->ntl; q.nlines = 3 * d->nz * d->NC; q.ny = d->ny; }
@@ -365,17 +399,20 @@ int build_tables(bm_batch_s* o)
 		}
 	for (size_t g = 0; g < o->gml.size(); g++)
 		for (int b : o->gml[g].meshes) {
+			if (col[(size_t)b]) continue;
 			const MlView v = mlayer_view(o->ml[b]);
 			o->tml[g].h.push_back(MlBatch{ v.S, v.K, v.NC, v.Ny, v.Sp });
 		}
 	for (size_t g = 0; g < o->gz.size(); g++)
 		for (int b : o->gz[g].meshes) {
+			if (col[(size_t)b]) continue;
 			bm_demag_s* d = o->dm[b];
 			PassBatch q{}; q.S = d->S; q.K = d->K; q.nz = d->nz; q.NC = d->NC; q.Ny = d->Ny; q.NYH = d->NYH; q.Sp = d->Sp;
 			o->tz[g].h.push_back(q);
 		}
 	for (size_t g = 0; g < o->gy2.size(); g++)
 		for (int b : o->gy2[g].meshes) {
+			if (col[(size_t)b]) continue;
 			bm_demag_s* d = o->dm[b];
 			PassBatch q{}; q.Sx = d->Sx; q.K = d->K; q.NC = d->NC; q.NYH = d->NYH; q.ntl = d->ntl; q.ny = d->ny;
 			o->ty2[g].h.push_back(q);
@@ -405,11 +442,13 @@ int build_tables(bm_batch_s* o)
 	for (auto& t : o->tml) at_ml.push_back(place(t));
 	std::vector<size_t> at_yz[2];
 	for (int q = 0; q < 2; q++) for (auto& t : o->tyz[q]) at_yz[q].push_back(place(t));
+	std::vector<size_t> at_col;
+	for (auto& g : o->gcol) at_col.push_back(place(g.t));
 	const size_t at_s0 = place(o->stage[0]), at_s1 = place(o->stage[1]), at_ch = place(o->choff);
 	if (hipMalloc(&o->dev_tables, std::max<size_t>(bytes, 256)) != hipSuccess) return fail(BM_ERR_NOMEM, "batch tables");
 	o->dev_bytes = bytes;
 	char* base = (char*)o->dev_tables;
-	for (auto& pc : pieces) BM_HIP(hipMemcpy(base + pc.first, pc.second.first, pc.second.second, hipMemcpyHostToDevice));
+	for (auto& pc : pieces) if (pc.second.second) BM_HIP(hipMemcpy(base + pc.first, pc.second.first, pc.second.second, hipMemcpyHostToDevice));
 	for (int par = 0; par < 2; par++) for (size_t g = 0; g < o->fwd[par].size(); g++) o->fwd[par][g].d = (FwdArgs*)(base + at_fwd[par][g]);
 	for (size_t g = 0; g < o->inv.size(); g++) o->inv[g].d = (PassBatch*)(base + at_inv[g]);
 	for (size_t g = 0; g < o->ty.size(); g++) o->ty[g].d = (PassBatch*)(base + at_y[g]);
@@ -417,6 +456,7 @@ int build_tables(bm_batch_s* o)
 	for (size_t g = 0; g < o->ty2.size(); g++) o->ty2[g].d = (PassBatch*)(base + at_y2[g]);
 	for (size_t g = 0; g < o->tml.size(); g++) o->tml[g].d = (MlBatch*)(base + at_ml[g]);
 	for (int q = 0; q < 2; q++) for (size_t g = 0; g < o->tyz[q].size(); g++) o->tyz[q][g].d = (PassBatch*)(base + at_yz[q][g]);
+	for (size_t g = 0; g < o->gcol.size(); g++) o->gcol[g].t.d = (ColBatch*)(base + at_col[g]);
 	o->stage[0].d = (StageArgs*)(base + at_s0);
 	o->stage[1].d = (StageArgs*)(base + at_s1);
 	o->choff.d = (int*)(base + at_ch);
@@ -456,25 +496,53 @@ template <typename F> int fan(bm_batch_s* o, size_t n, hipStream_t st, F&& launc
 	return rc;
 }
 
+// the groups of a pass that have meshes left for it
+template <class T> std::vector<size_t> live(const std::vector<Tab<T>>& tabs)
+{
+	std::vector<size_t> r;
+	for (size_t g = 0; g < tabs.size(); g++) if (!tabs[g].h.empty()) r.push_back(g);
+	return r;
+}
+
+// The middle passes of every mesh: first the meshes with one kernel for them (column, 2D y and
+// thin-mesh passes, all groups side by side), then the chain of separate passes.
+int middle_all(bm_batch_s* o, hipStream_t st)
+{
+	const std::vector<size_t> l2 = live(o->ty2), l4 = live(o->tyz[0]), l8 = live(o->tyz[1]), ly = live(o->ty), lz = live(o->tz), lm = live(o->tml);
+	const size_t nc = o->gcol.size();
+	int rc = fan(o, nc + l2.size() + l4.size() + l8.size(), st, [&](size_t q, hipStream_t s) {
+		if (q < nc) { auto& g = o->gcol[q]; return batch_col(g.Ny, g.kind, g.full, g.t.h.data(), g.t.d, (int)g.t.h.size(), s); }
+		if ((q -= nc) < l2.size()) {
+			const size_t g = l2[q];
+			return batch_y2d(o->gy2[g].size, o->gy2[g].full, o->gy2[g].sh[0], o->ty2[g].h.data(), o->ty2[g].d, (int)o->ty2[g].h.size(), o->ncu, s);
+		}
+		q -= l2.size();
+		const int w = q < l4.size() ? 0 : 1;
+		const size_t g = w ? l8[q - l4.size()] : l4[q];
+		return batch_yzy(o->gyz[w][g].size, w ? 8 : 4, o->gyz[w][g].sh[0], o->tyz[w][g].h.data(), o->tyz[w][g].d, (int)o->tyz[w][g].h.size(), o->ncu, s);
+	});
+	auto ypass = [&](int dir) {
+		return fan(o, ly.size(), st, [&](size_t q, hipStream_t s) {
+			const size_t g = ly[q];
+			return batch_y(o->gy[g].size, o->gy[g].full, dir, o->gy[g].sh[dir < 0 ? 0 : 1], o->ty[g].h.data(), o->ty[g].d, (int)o->ty[g].h.size(), o->ncu, s); });
+	};
+	if (!rc) rc = ypass(-1);
+	if (!rc) rc = fan(o, lz.size(), st, [&](size_t q, hipStream_t s) {
+		const size_t g = lz[q];
+		return batch_z(o->gz[g].size, o->gz[g].full, o->gz[g].sh[0], o->tz[g].h.data(), o->tz[g].d, (int)o->tz[g].h.size(), o->ncu, s); });
+	if (!rc) rc = fan(o, lm.size(), st, [&](size_t q, hipStream_t s) {
+		const size_t g = lm[q];
+		return batch_ml_mult(o->gml[g].size, o->gml[g].sh[0], o->tml[g].h.data(), o->tml[g].d, (int)o->tml[g].h.size(), o->ncu, s); });
+	if (!rc) rc = ypass(1);
+	return rc;
+}
+
 // One field evaluation + stage `step` for every mesh; input magnetisation M (parity 0) or Mb.
 int eval_all(bm_batch_s* o, int step, int par, hipStream_t st)
 {
 	int rc = fan(o, o->gx.size(), st, [&](size_t g, hipStream_t s) {
 		return batch_fwd_x(o->gx[g].size, o->gx[g].full, o->gx[g].sh[0], o->fwd[par][g].h.data(), o->fwd[par][g].d, (int)o->fwd[par][g].h.size(), o->ncu, s); });
-	if (!rc) rc = fan(o, o->gy.size(), st, [&](size_t g, hipStream_t s) {
-		return batch_y(o->gy[g].size, o->gy[g].full, -1, o->gy[g].sh[0], o->ty[g].h.data(), o->ty[g].d, (int)o->ty[g].h.size(), o->ncu, s); });
-	if (!rc) rc = fan(o, o->gz.size(), st, [&](size_t g, hipStream_t s) {
-		return batch_z(o->gz[g].size, o->gz[g].full, o->gz[g].sh[0], o->tz[g].h.data(), o->tz[g].d, (int)o->tz[g].h.size(), o->ncu, s); });
-	if (!rc) rc = fan(o, o->gml.size(), st, [&](size_t g, hipStream_t s) {
-		return batch_ml_mult(o->gml[g].size, o->gml[g].sh[0], o->tml[g].h.data(), o->tml[g].d, (int)o->tml[g].h.size(), o->ncu, s); });
-	if (!rc) rc = fan(o, o->gy.size(), st, [&](size_t g, hipStream_t s) {
-		return batch_y(o->gy[g].size, o->gy[g].full, 1, o->gy[g].sh[1], o->ty[g].h.data(), o->ty[g].d, (int)o->ty[g].h.size(), o->ncu, s); });
-	if (!rc) rc = fan(o, o->gy2.size(), st, [&](size_t g, hipStream_t s) {
-		return batch_y2d(o->gy2[g].size, o->gy2[g].full, o->gy2[g].sh[0], o->ty2[g].h.data(), o->ty2[g].d, (int)o->ty2[g].h.size(), o->ncu, s); });
-	for (int q = 0; q < 2 && !rc; q++)
-		rc = fan(o, o->gyz[q].size(), st, [&](size_t g, hipStream_t s) {
-			return batch_yzy(o->gyz[q][g].size, q ? 8 : 4, o->gyz[q][g].sh[0], o->tyz[q][g].h.data(), o->tyz[q][g].d, (int)o->tyz[q][g].h.size(),
-				o->ncu, s); });
+	if (!rc) rc = middle_all(o, st);
 	if (!rc) rc = fan(o, o->gx.size(), st, [&](size_t g, hipStream_t s) {
 		return batch_inv_x_planar(o->gx[g].size, o->gx[g].full, o->gx[g].sh[1], o->inv[g].h.data(), o->inv[g].d, (int)o->inv[g].h.size(), o->ncu, s); });
 	if (!rc) rc = batch_stage(o->mcode, step, o->stage[par].d, o->nb, o->choff.d, o->choff.h.back(), st);
@@ -483,9 +551,10 @@ int eval_all(bm_batch_s* o, int step, int par, hipStream_t st)
 
 // Autotuner: for every pass-size group and pass, time each candidate launch shape (five
 // launches after a warm-up, HIP events) on the group's real tables and keep the fastest.
-// Candidates: x passes tile factor {1, 2} x workgroups per CU {1, 2, 4}, and the half-height
-// tile at {2, 4, 8} per CU where the row length has one; y passes {4, 8, 16};
-// z pass {1, 2, 4}; 2D y pass {4, 8, 16}; multilayer product {4, 8, 16}.  Only the FFT passes
+// Candidates: x passes the default, tile factor {1, 2} x workgroups per CU {1, 2, 4}, and the
+// half-height tile at {2, 4, 8} per CU where the row length has one; y passes {4, 8, 16};
+// z pass {1, 2, 4}; 2D y pass {4, 8, 16}; multilayer product {4, 8, 16}.  Then the middle passes
+// as a whole, tuned, against their default shapes (with which meshes take the column pass).  Only the FFT passes
 // run (their inputs are recomputed from M by every evaluation), so the state is untouched.
 int autotune(bm_batch_s* o, hipStream_t st)
 {
@@ -515,6 +584,7 @@ int autotune(bm_batch_s* o, hipStream_t st)
 		G.sh[slot] = best; G.us[slot] = bt;
 	};
 	std::vector<LaunchShape> cx, cxh, cy, cz;
+	cx.push_back(LaunchShape{});
 	for (int f : { 1, 2 }) for (int pc : { 1, 2, 4 }) cx.push_back(LaunchShape{ f, pc });
 	// with the half-height tile (twice the work items for small meshes) where the length has one
 	cxh = cx;
@@ -522,7 +592,7 @@ int autotune(bm_batch_s* o, hipStream_t st)
 	for (int pc : { 4, 8, 16 }) cy.push_back(LaunchShape{ 0, pc });
 	for (int pc : { 1, 2, 4 }) cz.push_back(LaunchShape{ 0, pc });
 	// the launch shapes crossed with every radix schedule of the pass length n
-	std::vector<LaunchShape> cx1;
+	std::vector<LaunchShape> cx1(1, LaunchShape{});
 	for (int pc : { 1, 2, 4 }) cx1.push_back(LaunchShape{ 1, pc });
 	// the launch shapes crossed with every radix schedule of the pass length n (periodic
 	// groups: the default schedule only)
@@ -532,6 +602,8 @@ int autotune(bm_batch_s* o, hipStream_t st)
 		for (int v = 0; v < nv; v++) for (LaunchShape c : base) { c.radix = v; r.push_back(c); }
 		return r;
 	};
+	o->no_col = true;
+	rc = build_tables(o);
 	for (size_t g = 0; g < o->gx.size() && !rc; g++) {
 		Group& G = o->gx[g];
 		const std::vector<LaunchShape>& cands = G.full ? cx1 : x_half_tile_ok(G.size) ? cxh : cx;
@@ -560,6 +632,18 @@ int autotune(bm_batch_s* o, hipStream_t st)
 			Group& G = o->gyz[q][g];
 			pick(G, 0, cy, false, [&] { return batch_yzy(G.size, q ? 8 : 4, G.sh[0], o->tyz[q][g].h.data(), o->tyz[q][g].d, (int)o->tyz[q][g].h.size(), o->ncu, st); });
 		}
+	if (!rc) {
+		const double tuned = timed([&] { return middle_all(o, st); });
+		o->no_col = false;
+		std::vector<std::pair<Group*, Group>> keep;
+		for (std::vector<Group>* gs : { &o->gy, &o->gz, &o->gy2, &o->gml, &o->gyz[0], &o->gyz[1] })
+			for (Group& G : *gs) { keep.push_back({ &G, G }); G.sh[0] = G.sh[1] = LaunchShape{}; }
+		rc = build_tables(o);
+		const double plain = rc ? -1 : timed([&] { return middle_all(o, st); });
+		if (plain >= 0 && plain < tuned) { for (auto& k : keep) k.first->us[0] = k.first->us[1] = plain; }   // the whole middle's time
+		else for (auto& k : keep) *k.first = k.second;
+	}
+	o->no_col = false;
 	if (!rc) rc = build_tables(o);
 	(void)hipEventDestroy(e0);
 	(void)hipEventDestroy(e1);
@@ -984,7 +1068,7 @@ extern "C" int bm_batch_set_schedule(bm_batch_t o, const char* pass, int size, i
 	if (o->exec) { (void)hipGraphExecDestroy(o->exec); o->exec = nullptr; }
 	if (o->graph) { (void)hipGraphDestroy(o->graph); o->graph = nullptr; }
 	int rc;
-	if (x && (rc = build_tables(o))) return rc;
+	if ((rc = build_tables(o))) return rc;
 	o->autotune = false;
 	o->tuned = true;
 	return BM_OK;

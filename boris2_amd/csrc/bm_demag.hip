@@ -352,9 +352,9 @@ __global__ void __launch_bounds__(kBlock) k_z(float2* __restrict__ S, const floa
 			const float kxx = kr[kzr], kyy = kr[KR * NZH + kzr], kzz = kr[2 * KR * NZH + kzr];
 			const float kxy = sy * kr[3 * KR * NZH + kzr], kxz = sz * kr[4 * KR * NZH + kzr], kyz = sy * sz * kr[5 * KR * NZH + kzr];
 			C2<float> mx = v[0][e], my = v[1][e], mz = v[2][e];
-			v[0][e] = mk(kxx * mx.x + kxy * my.x + kxz * mz.x, kxx * mx.y + kxy * my.y + kxz * mz.y);
-			v[1][e] = mk(kxy * mx.x + kyy * my.x + kyz * mz.x, kxy * mx.y + kyy * my.y + kyz * mz.y);
-			v[2][e] = mk(kxz * mx.x + kyz * my.x + kzz * mz.x, kxz * mx.y + kyz * my.y + kzz * mz.y);
+			v[0][e] = lin3(kxx, mx, kxy, my, kxz, mz);
+			v[1][e] = lin3(kxy, mx, kyy, my, kyz, mz);
+			v[2][e] = lin3(kxz, mx, kyz, my, kzz, mz);
 		}
 		fft3<PK, 1, float>(v[0], v[1], v[2], lds + col, lds + NZ * CY + col, lds + 2 * NZ * CY + col, CY, t, tw);
 		if (ok) {
@@ -412,8 +412,8 @@ __global__ void __launch_bounds__(BS) k_y2d(float2* __restrict__ Sx, const float
 			const size_t ki = (size_t)kxs * NYH + kyr;
 			const float kxx = K[ki], kyy = K[kq + ki], kzz = K[2 * kq + ki], kxy = sy * K[3 * kq + ki];
 			C2<float> mx = v[0][e], my = v[1][e], mz = v[2][e];
-			v[0][e] = mk(kxx * mx.x + kxy * my.x, kxx * mx.y + kxy * my.y);
-			v[1][e] = mk(kxy * mx.x + kyy * my.x, kxy * mx.y + kyy * my.y);
+			v[0][e] = lin2(kxx, mx, kxy, my);
+			v[1][e] = lin2(kxy, mx, kyy, my);
 			v[2][e] = mk(kzz * mz.x, kzz * mz.y);
 		}
 		fft3<PK, 1, float>(v[0], v[1], v[2], b0, b0 + LP * LL, b0 + 2 * LP * LL, 1, t, tw);
@@ -865,9 +865,9 @@ __global__ void __launch_bounds__(BS) k_yzy(float2* __restrict__ Sx, const float
 					const float kxx = kb[kzr], kyy = kb[kq + kzr], kzz = kb[2 * kq + kzr];
 					const float kxy = sy * kb[3 * kq + kzr], kxz = sz * kb[4 * kq + kzr], kyz = sy * sz * kb[5 * kq + kzr];
 					const C2<float> mx = u[0][kz], my = u[1][kz], mz = u[2][kz];
-					u[0][kz] = mk(kxx * mx.x + kxy * my.x + kxz * mz.x, kxx * mx.y + kxy * my.y + kxz * mz.y);
-					u[1][kz] = mk(kxy * mx.x + kyy * my.x + kyz * mz.x, kxy * mx.y + kyy * my.y + kyz * mz.y);
-					u[2][kz] = mk(kxz * mx.x + kyz * my.x + kzz * mz.x, kxz * mx.y + kyz * my.y + kzz * mz.y);
+					u[0][kz] = lin3(kxx, mx, kxy, my, kxz, mz);
+					u[1][kz] = lin3(kxy, mx, kyy, my, kyz, mz);
+					u[2][kz] = lin3(kxz, mx, kyz, my, kzz, mz);
 				}
 #pragma unroll
 				for (int c = 0; c < 3; c++) {
@@ -926,9 +926,9 @@ __global__ void __launch_bounds__(BS) k_yzy(float2* __restrict__ Sx, const float
 				const float kxx = kb[kzr], kyy = kb[kq + kzr], kzz = kb[2 * kq + kzr];
 				const float kxy = sy * kb[3 * kq + kzr], kxz = sz * kb[4 * kq + kzr], kyz = sy * sz * kb[5 * kq + kzr];
 				const C2<float> mx = u[0][kz], my = u[1][kz], mz = u[2][kz];
-				u[0][kz] = mk(kxx * mx.x + kxy * my.x + kxz * mz.x, kxx * mx.y + kxy * my.y + kxz * mz.y);
-				u[1][kz] = mk(kxy * mx.x + kyy * my.x + kyz * mz.x, kxy * mx.y + kyy * my.y + kyz * mz.y);
-				u[2][kz] = mk(kxz * mx.x + kyz * my.x + kzz * mz.x, kxz * mx.y + kyz * my.y + kzz * mz.y);
+				u[0][kz] = lin3(kxx, mx, kxy, my, kxz, mz);
+				u[1][kz] = lin3(kxy, mx, kyy, my, kyz, mz);
+				u[2][kz] = lin3(kxz, mx, kyz, my, kzz, mz);
 			}
 #pragma unroll
 			for (int c = 0; c < 3; c++) {
@@ -1013,6 +1013,16 @@ bool yzy_ok(const bm_demag_s* d)
 #undef C_
 	}
 	return false;
+}
+
+// The column pass serves this mesh (open z) and is the better one: from N.y = 1024 with N.z = 4 the
+// thin-mesh pass, which keeps both planes in registers, is faster (512x512x2 61.0 -> 57.0 us,
+// 768x512x2 93 -> 81; 1024x256x2 57.5 -> 58.8, 256x256x2 23.8 -> 26.7).
+bool use_col(const bm_demag_s* d)
+{
+	if (!d->yzy || d->full[2] || pass_tune().y_radix || pass_tune().y_percu || pass_tune().z_radix || pass_tune().z_percu) return false;
+	if (yzy_ok(d) && (d->yzy == 2 || d->Ny >= 1024)) return false;
+	return col_ok(d->Ny, d->Nz, d->nz, d->NC, d->ncu);
 }
 
 int launch_yzy(const bm_demag_s* d, hipStream_t st)
@@ -1196,6 +1206,13 @@ int bm::demag_mid(bm_demag_s* d, hipStream_t st)
 {
 	const int nlines = 3 * d->nz * d->NC;
 	int rc;
+	if (use_col(d)) {
+		// the middle passes as one, timed as the 2D y or the z pass
+		prof_mark_begin(d->is2d ? PK_Y2D : PK_Z, st);
+		rc = launch_col(d->Ny, d->Nz, d->full[1], d->Sx, d->K, nullptr, d->nz, d->NC, d->NYH, d->ntl, d->full[1] ? d->Ny : d->ny, 0, st);
+		prof_mark_end(d->is2d ? PK_Y2D : PK_Z, st);
+		return rc;
+	}
 	if (d->is2d) {
 		prof_mark_begin(PK_Y2D, st);
 		rc = launch_y2d(d->Ny, d->full[1], d->Sx, d->K, d->NC, d->NYH, d->ntl, d->full[1] ? d->Ny : d->ny, d->ncu, st);
@@ -1744,6 +1761,7 @@ int bm::batch_y2d(int Ny, bool full, LaunchShape sh, const PassBatch* h_tab, con
 }
 
 bool bm::demag_yzy(const bm_demag_s* d) { return yzy_ok(d); }
+bool bm::demag_col(const bm_demag_s* d) { return use_col(d); }
 
 int bm::batch_yzy(int Ny, int Nz, LaunchShape sh, const PassBatch* h_tab, const PassBatch* d_tab, int nb, int ncu, hipStream_t st)
 {

@@ -34,6 +34,14 @@ template <typename T> __device__ __forceinline__ C2<T> conj(C2<T> a) { return mk
 // multiply by DIR*i  (DIR = -1 forward, +1 inverse)
 template <int DIR, typename T> __device__ __forceinline__ C2<T> mul_di(C2<T> a) { return DIR < 0 ? mk(a.y, -a.x) : mk(-a.y, a.x); }
 
+// a x + b y and a x + b y + c z (real coefficients) with the roundings written out, so that the
+// kernels that take each other's place for the demag product give the same bits
+template <typename T> __device__ __forceinline__ C2<T> lin2(T a, C2<T> x, T b, C2<T> y) { return mk(fma(a, x.x, b * y.x), fma(a, x.y, b * y.y)); }
+template <typename T> __device__ __forceinline__ C2<T> lin3(T a, C2<T> x, T b, C2<T> y, T c, C2<T> z)
+{
+	return mk(fma(a, x.x, fma(b, y.x, c * z.x)), fma(a, x.y, fma(b, y.y, c * z.y)));
+}
+
 // ----------------------------------------------------------------------------------------
 // Radix plans.  E = values per thread; each radix divides E; the first radix is even so a
 // zero upper half of the input maps onto whole zero inputs of the first butterflies.

@@ -61,8 +61,9 @@ struct bm_demag_s {
 	int ncu = 256;
 	bool row_wave = false;    // integrator row kernel at nx = 512: the wave-independent variant
 	                          // (BM_ROW_WAVE=1 at creation; measured slower, kept for tests)
-	int yzy = 1;              // fused y, z, y pass for thin meshes (N.z 4 or 8): 1 for N.z = 4 from
-	                          // 128 x 128 cells per plane, 2 always, 0 never (BM_YZY at creation)
+	int yzy = 1;              // fused middle passes (BM_YZY at creation): 1 the column pass where it serves
+	                          // the mesh, else or from N.y = 1024 with N.z = 4 the thin-mesh pass; 2 the
+	                          // thin-mesh pass wherever it can (N.z 4 or 8); 0 the separate passes
 };
 
 namespace bm {
@@ -120,6 +121,13 @@ int launch_inv_xs(int HX, bool full, int mode, const float2* Sx, float* out, int
 	const float* M, double* epart, int nx, int zoff, int nzl);
 int batch_fwd_xs(int HX, bool full, const FwdArgs* h_tab, const FwdArgs* d_tab, int nb, hipStream_t st);
 int batch_inv_xs_planar(int HX, bool full, const struct PassBatch* h_tab, const struct PassBatch* d_tab, int nb, hipStream_t st);
+// The middle passes as one kernel per kx column group (bm_col.hip): whether it serves N.y, kind (N.z
+// of a 3D mesh, 1: 2D, 0: layers), P planes or layers and NC columns, and its launcher (full:
+// periodic y; tr: the layers' transposed product).
+struct ColBatch { float2* Sx; const float* K; int P, NC, NYH, ntl, nyd; };   // one mesh or stack of a batched launch
+bool col_ok(int Ny, int kind, int P, int NC, int ncu);
+int batch_col(int Ny, int kind, bool full, const ColBatch* h_tab, const ColBatch* d_tab, int nb, hipStream_t st);
+int launch_col(int Ny, int kind, bool full, float2* Sx, const float* K, const int* kidx, int P, int NC, int NYH, int ntl, int nyd, int tr, hipStream_t st);
 // Per-mesh arguments of the other passes in a batched launch (the fields each pass uses;
 // the y passes take ny as the data rows of a line).
 struct PassBatch {
@@ -177,5 +185,7 @@ int batch_y2d(int Ny, bool full, LaunchShape sh, const PassBatch* h_tab, const P
 // thin meshes (N.z 4 or 8, open y and z, a power-of-two N.y with a fitting schedule): the y, z,
 // y passes as one kernel that never writes the full spectra; demag_yzy: the handle takes it
 bool demag_yzy(const bm_demag_s* d);
+// the handle's middle passes run as the column pass
+bool demag_col(const bm_demag_s* d);
 int batch_yzy(int Ny, int Nz, LaunchShape sh, const PassBatch* h_tab, const PassBatch* d_tab, int nb, int ncu, hipStream_t st);
 }

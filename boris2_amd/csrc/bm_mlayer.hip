@@ -1140,6 +1140,15 @@ static int ml_convolute(bm_mlayer_s* m, const float* M, float* out, int mode, hi
 	const int L = m->L, nlines = 3 * L * m->NC;
 	const bool fx = m->pbc[0] > 0, fy = m->pbc[1] > 0;
 	int rc = bm::pass_fwd_x(m->xs, M, m->Sx, m->ny, L, m->ntl, m->ncu, st, fx);
+	if (rc == BM_OK && !m->Kc && bm::col_ok(m->Ny, 0, L, m->NC, m->ncu)) {
+		// the y passes and the product as one, timed as the product
+		bm::prof_mark_begin(bm::PK_ML_MULT, st);
+		rc = bm::launch_col(m->Ny, 0, fy, m->Sx, m->K, m->kidx, L, m->NC, m->NYH, m->ntl, fy ? m->Ny : m->ny, tr, st);
+		bm::prof_mark_end(bm::PK_ML_MULT, st);
+		const float scale = (float)(1.0 / ((double)m->Nx * m->Ny));
+		if (rc == BM_OK) rc = bm::pass_inv_x(m->xs, mode, m->Sx, out, m->ny, L, m->ntl, scale, m->ncu, st, fx);
+		return rc;
+	}
 	if (rc == BM_OK) rc = bm::pass_y(m->Ny, -1, m->S, m->Sx, nlines, m->Sp, m->NC, m->ntl, m->ncu, st, fy);
 	if (rc == BM_OK) {
 		bm::prof_mark_begin(bm::PK_ML_MULT, st);

@@ -1,0 +1,68 @@
+"""The middle passes as one kernel per kx column (bm_col): every line length and z length it serves,
+at the fewest and most planes or layers of each, open and periodic y, against the FP64 oracle (the
+field's parity bar, 1e-6 relative L2), and against the separate passes, whose arithmetic it repeats
+(FP32 rounding: 5e-7; a field evaluation's own error is below 2e-7)."""
+import numpy as np
+import pytest
+import torch
+
+from boris2_amd import api
+import oracle_lib as O
+
+pytestmark = pytest.mark.gpu
+H = (4e-9, 4e-9, 4e-9)
+
+
+def rel(a, b):
+    return np.linalg.norm(a - b) / np.linalg.norm(b)
+
+
+def nz_open(nz):
+    N = 1
+    while nz > 1 and N < 2 * nz:
+        N *= 2
+    return N
+
+
+# N.y = 4 ... 1024 (2D); N.z = 4 (nz 2), 8 (3, 4), 16 (5, 8), 32 (9, 16); column counts around the
+# lanes of a wave and beyond the compute units
+OPEN = [(6, 2, 1), (4, 3, 1), (8, 4, 1), (12, 6, 1), (16, 8, 1), (2, 12, 1), (24, 16, 1), (32, 24, 1), (64, 32, 1), (48, 48, 1), (8, 64, 1),
+        (16, 96, 1), (12, 128, 1), (6, 192, 1), (4, 256, 1), (6, 384, 1), (4, 512, 1), (8, 100, 1),
+        (8, 8, 2), (16, 2, 3), (12, 24, 4), (6, 96, 4), (4, 256, 4), (8, 48, 5), (6, 64, 8), (4, 250, 8), (2, 384, 5), (8, 16, 9), (12, 64, 16),
+        (6, 128, 16), (2, 48, 12), (260, 12, 8)]
+
+
+@pytest.mark.parametrize("n", OPEN)
+def test_open(gpu, monkeypatch, n):
+    M0 = api.random_magnetisation(n[0] * n[1] * n[2], 8e5, 2).astype(np.float32)
+    M = torch.from_numpy(M0).cuda()
+    d = api.Demag(n, H)
+    got = d.convolute(M).cpu().numpy().astype(np.float64)
+    ref = O.OracleDemag(n, H, Nz_override=nz_open(n[2]))(M0.astype(np.float64))
+    assert rel(got, ref) <= 1e-6
+    monkeypatch.setenv("BM_YZY", "0")
+    s = api.Demag(n, H)
+    assert rel(got, s.convolute(M).cpu().numpy().astype(np.float64)) <= 5e-7
+    d.close(); s.close()
+
+
+@pytest.mark.parametrize("n,pbc", [((8, 12, 1), (0, 3, 0)), ((16, 64, 4), (2, 2, 0)), ((8, 96, 8), (0, 2, 0)), ((4, 256, 2), (0, 2, 0)), ((6, 32, 16), (0, 2, 0))])
+def test_periodic_y(gpu, n, pbc):
+    M0 = api.random_magnetisation(n[0] * n[1] * n[2], 8e5, 4).astype(np.float32)
+    d = api.Demag(n, H, pbc)
+    ref = O.OracleDemag(n, H, Nz_override=nz_open(n[2]), pbc=pbc)(M0.astype(np.float64))
+    assert rel(d.convolute(torch.from_numpy(M0).cuda()).cpu().numpy().astype(np.float64), ref) <= 1e-6
+    d.close()
+
+
+# layers of one thickness and of two; as many as 512 threads hold, then 1024
+@pytest.mark.parametrize("nx,ny,L,pbc", [(8, 8, 1, (0, 0)), (16, 24, 2, (0, 0)), (12, 64, 3, (0, 0)), (6, 256, 4, (0, 0)), (8, 64, 16, (0, 0)), (4, 128, 9, (0, 0)),
+                                         (4, 128, 16, (0, 0)), (4, 512, 2, (0, 0)), (4, 512, 3, (0, 0)), (6, 384, 3, (0, 0)), (8, 32, 5, (0, 2)), (16, 64, 12, (2, 2))])
+def test_layers(gpu, nx, ny, L, pbc):
+    hz = [4e-9 if l % 3 else 8e-9 for l in range(L)]
+    z0 = [12e-9 * l for l in range(L)]
+    M0 = api.random_magnetisation(nx * ny * L, 8e5, 6).astype(np.float32)
+    d = api.MultiLayerDemag(nx, ny, 4e-9, 4e-9, hz, z0, pbc)
+    ref = O.OracleMLayer(nx, ny, 4e-9, 4e-9, np.array(hz), np.array(z0), pbc)(M0.astype(np.float64))
+    assert rel(d.convolute(torch.from_numpy(M0).cuda()).cpu().numpy().astype(np.float64), np.asarray(ref).reshape(-1, 3)) <= 1e-6
+    d.close()
