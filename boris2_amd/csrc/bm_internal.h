@@ -140,6 +140,10 @@ struct PassBatch {
 int mlayer_planar(bm_mlayer_s* m, const float* M, float* H3n, hipStream_t st);
 // the transposed operator N^T (the adjoint of the multilayered convolution), planar output
 int mlayer_planar_transposed(bm_mlayer_s* m, const float* M, float* H3n, hipStream_t st);
+// its passes: x R2C of M (AoS, all layers) into the handle's spectra, and the middle (product; tr: of
+// the transposed operator)
+int mlayer_fwd_x(bm_mlayer_s* m, const float* M, hipStream_t st);
+int mlayer_mid(bm_mlayer_s* m, hipStream_t st, int tr = 0);
 void mlayer_dims(const bm_mlayer_s* m, int* L, int* nx, int* ny, double* hz);
 // the handle's layers are meshes of their own on a common grid (bm_mlayer_create_meshes, or a
 // size without a plan): only the convolution calls take it

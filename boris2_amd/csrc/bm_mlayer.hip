@@ -1133,31 +1133,41 @@ extern "C" int bm_mlayer_destroy(bm_mlayer_t m)
 	return BM_OK;
 }
 
-// The convolution (tr: its transpose) into out with the final x C2R in `mode` (0 planar
-// set, 1 AoS set, 2 AoS add).
-static int ml_convolute(bm_mlayer_s* m, const float* M, float* out, int mode, hipStream_t st, int tr = 0)
+int bm::mlayer_fwd_x(bm_mlayer_s* m, const float* M, hipStream_t st)
+{
+	return bm::pass_fwd_x(m->xs, M, m->Sx, m->ny, m->L, m->ntl, m->ncu, st, m->pbc[0] > 0);
+}
+
+int bm::mlayer_mid(bm_mlayer_s* m, hipStream_t st, int tr)
 {
 	const int L = m->L, nlines = 3 * L * m->NC;
-	const bool fx = m->pbc[0] > 0, fy = m->pbc[1] > 0;
-	int rc = bm::pass_fwd_x(m->xs, M, m->Sx, m->ny, L, m->ntl, m->ncu, st, fx);
-	if (rc == BM_OK && !m->Kc && bm::col_ok(m->Ny, 0, L, m->NC, m->ncu)) {
+	const bool fy = m->pbc[1] > 0;
+	int rc;
+	if (!m->Kc && bm::col_ok(m->Ny, 0, L, m->NC, m->ncu)) {
 		// the y passes and the product as one, timed as the product
 		bm::prof_mark_begin(bm::PK_ML_MULT, st);
 		rc = bm::launch_col(m->Ny, 0, fy, m->Sx, m->K, m->kidx, L, m->NC, m->NYH, m->ntl, fy ? m->Ny : m->ny, tr, st);
 		bm::prof_mark_end(bm::PK_ML_MULT, st);
-		const float scale = (float)(1.0 / ((double)m->Nx * m->Ny));
-		if (rc == BM_OK) rc = bm::pass_inv_x(m->xs, mode, m->Sx, out, m->ny, L, m->ntl, scale, m->ncu, st, fx);
 		return rc;
 	}
-	if (rc == BM_OK) rc = bm::pass_y(m->Ny, -1, m->S, m->Sx, nlines, m->Sp, m->NC, m->ntl, m->ncu, st, fy);
+	rc = bm::pass_y(m->Ny, -1, m->S, m->Sx, nlines, m->Sp, m->NC, m->ntl, m->ncu, st, fy);
 	if (rc == BM_OK) {
 		bm::prof_mark_begin(bm::PK_ML_MULT, st);
 		rc = launch_ml_mult(L, m->S, m->S2, m->K, m->kidx, m->NC, m->Ny, m->Sp, m->ncu, st, tr, m->Kc, m->kcoff);
 		bm::prof_mark_end(bm::PK_ML_MULT, st);
 	}
 	if (rc == BM_OK) rc = bm::pass_y(m->Ny, 1, m->Sout(), m->Sx, nlines, m->Sp, m->NC, m->ntl, m->ncu, st, fy);
+	return rc;
+}
+
+// The convolution (tr: its transpose) into out with the final x C2R in `mode` (0 planar
+// set, 1 AoS set, 2 AoS add).
+static int ml_convolute(bm_mlayer_s* m, const float* M, float* out, int mode, hipStream_t st, int tr = 0)
+{
+	int rc = bm::mlayer_fwd_x(m, M, st);
+	if (rc == BM_OK) rc = bm::mlayer_mid(m, st, tr);
 	const float scale = (float)(1.0 / ((double)m->Nx * m->Ny));
-	if (rc == BM_OK) rc = bm::pass_inv_x(m->xs, mode, m->Sx, out, m->ny, L, m->ntl, scale, m->ncu, st, fx);
+	if (rc == BM_OK) rc = bm::pass_inv_x(m->xs, mode, m->Sx, out, m->ny, m->L, m->ntl, scale, m->ncu, st, m->pbc[0] > 0);
 	return rc;
 }
 

@@ -219,6 +219,10 @@ __global__ void __launch_bounds__(kXBlock) k_roww(StageArgs a, float2* Sx, int n
 	if (stage_has_lte<METHOD, STEP>()) block_max_to<kXBlock>(lte_loc, a.lte);
 }
 
+// What the row kernel works on: the x-side spectra of nz planes of ny rows (a mesh's, or a stack's
+// layers); row_wave as bm_demag_s.
+struct RowGeom { float2* Sx; int nx, ny, nz, ntl, ncu; bool row_wave; };
+
 // Grid of the row kernel: a multiple of 8 blocks (the XCD split needs it), about two per CU.
 inline int row_grid(int nwork, int ncu)
 {
@@ -227,24 +231,26 @@ inline int row_grid(int nwork, int ncu)
 }
 
 template <int METHOD, int STEP, bool R2C>
-int launch_row_t(const bm_demag_s* d, const StageArgs& a, float scale, hipStream_t st)
+int launch_row_t(const RowGeom& d, const StageArgs& a, float scale, hipStream_t st)
 {
-	if (d->nx == 512 && d->row_wave) {
+	if (d.nx == 512 && d.row_wave) {
 		constexpr int TY = kLT;
-		const int nt = (d->ny + TY - 1) / TY;
-		hipLaunchKernelGGL((k_roww<512, METHOD, STEP, R2C>), dim3(row_grid(d->nz * nt, d->ncu)), dim3(kXBlock), 0, st, a, d->Sx, d->ntl, nt, scale);
+		const int nt = (d.ny + TY - 1) / TY;
+		hipLaunchKernelGGL((k_roww<512, METHOD, STEP, R2C>), dim3(row_grid(d.nz * nt, d.ncu)), dim3(kXBlock), 0, st, a, d.Sx, d.ntl, nt, scale);
 		return BM_OK;
 	}
-	switch (d->nx) {
+	switch (d.nx) {
 #define C_(V_) case V_: { \
-	if constexpr (xs_ok<V_>()) if (xs_few_rows(V_, d->ny, d->nz, d->ncu, true)) { \
-		const int ns = (d->ny + XSplit<V_>::RP - 1) / XSplit<V_>::RP, g = d->nz * ns; \
-		hipLaunchKernelGGL((k_rows<V_, METHOD, STEP, R2C>), dim3((g + 7) / 8 * 8), dim3(XSplit<V_>::BS), 0, st, a, d->Sx, d->ntl, ns, scale); \
+	if constexpr (xs_ok<V_>()) if (xs_few_rows(V_, d.ny, d.nz, d.ncu, true)) { \
+		const int ns = (d.ny + XSplit<V_>::RP - 1) / XSplit<V_>::RP, g = d.nz * ns; \
+		const dim3 gd((g + 7) / 8 * 8), bd(XSplit<V_>::BS); \
+		if (a.layered) hipLaunchKernelGGL((k_rows<V_, METHOD, STEP, R2C, true>), gd, bd, 0, st, a, d.Sx, d.ntl, ns, scale); \
+		else hipLaunchKernelGGL((k_rows<V_, METHOD, STEP, R2C, false>), gd, bd, 0, st, a, d.Sx, d.ntl, ns, scale); \
 		return BM_OK; \
 	} \
 	if constexpr (!xs_row_only<V_>()) { \
-		constexpr int TY = XTile<V_>::v; const int nt = (d->ny + TY - 1) / TY; \
-		hipLaunchKernelGGL((k_row<V_, TY, METHOD, STEP, R2C>), dim3(row_grid(d->nz * nt, d->ncu)), dim3(kXBlock), 0, st, a, d->Sx, d->ntl, nt, scale); \
+		constexpr int TY = XTile<V_>::v; const int nt = (d.ny + TY - 1) / TY; \
+		hipLaunchKernelGGL((k_row<V_, TY, METHOD, STEP, R2C>), dim3(row_grid(d.nz * nt, d.ncu)), dim3(kXBlock), 0, st, a, d.Sx, d.ntl, nt, scale); \
 		return BM_OK; \
 	} } break;
 	BM_FOR_ROW_SIZES(C_)
@@ -254,8 +260,8 @@ int launch_row_t(const bm_demag_s* d, const StageArgs& a, float scale, hipStream
 }
 
 // per-method launchers (one translation unit each)
-int launch_row_rkdp(const bm_demag_s* d, const StageArgs& a, int step, float scale, hipStream_t st);
-int launch_row_rk4(const bm_demag_s* d, const StageArgs& a, int step, float scale, hipStream_t st);
-int launch_row_heun(const bm_demag_s* d, const StageArgs& a, int mcode, int step, float scale, hipStream_t st);
+int launch_row_rkdp(const RowGeom& d, const StageArgs& a, int step, float scale, hipStream_t st);
+int launch_row_rk4(const RowGeom& d, const StageArgs& a, int step, float scale, hipStream_t st);
+int launch_row_heun(const RowGeom& d, const StageArgs& a, int mcode, int step, float scale, hipStream_t st);
 
 } // namespace bm

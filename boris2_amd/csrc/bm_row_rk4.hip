@@ -1,7 +1,7 @@
 // Row kernels of the RK4 stages.
 #include "bm_row.h"
 
-int bm::launch_row_rk4(const bm_demag_s* d, const StageArgs& a, int step, float scale, hipStream_t st)
+int bm::launch_row_rk4(const RowGeom& d, const StageArgs& a, int step, float scale, hipStream_t st)
 {
 	switch (step) {
 	case 0: return launch_row_t<M_RK4, 0, true>(d, a, scale, st);

@@ -2,7 +2,7 @@
 // advance that follows it runs in the forward x pass of the convolution).
 #include "bm_row.h"
 
-int bm::launch_row_rkdp(const bm_demag_s* d, const StageArgs& a, int step, float scale, hipStream_t st)
+int bm::launch_row_rkdp(const RowGeom& d, const StageArgs& a, int step, float scale, hipStream_t st)
 {
 	switch (step) {
 	case 0: return launch_row_t<M_RKDP, 0, false>(d, a, scale, st);

@@ -339,11 +339,14 @@ __device__ __forceinline__ void stage_cell(const StageArgs& a, F3 Ha, size_t idx
 
 // Cells i0 = 2k and i0 + 1 of row (j, k) for the row kernel (nx even, so both exist).  Row
 // and plane boundaries are uniform over a row, so only the x ends take a per-lane select.
-// Returns the output magnetisation of both cells.
-template <int METHOD, int STEP>
+// Returns the output magnetisation of both cells.  LAY: the mesh is a layer stack (a row lies in one
+// layer).
+template <int METHOD, int STEP, bool LAY = false>
 __device__ __forceinline__ P6 stage_pair(const StageArgs& a, size_t idx, int i0, int j, int k, P6 m, P6 Hd, float& lte_loc)
 {
-	const float2 Ms = a.Ms_map ? *reinterpret_cast<const float2*>(a.Ms_map + idx) : make_float2(a.Ms, a.Ms);
+	// a stack's Ms map and extra field are read by single cells (any 4-byte aligned array)
+	const float2 Ms = !a.Ms_map ? make_float2(a.Ms, a.Ms) : LAY ? make_float2(a.Ms_map[idx], a.Ms_map[idx + 1])
+		: *reinterpret_cast<const float2*>(a.Ms_map + idx);
 	F3 lap0{ 0.f, 0.f, 0.f }, lap1{ 0.f, 0.f, 0.f };
 	if (a.modules & BM_MOD_EXCHANGE) {
 		// x: the two cells are each other's neighbours; clamped loads keep the ends branch-free
@@ -359,19 +362,30 @@ __device__ __forceinline__ P6 stage_pair(const StageArgs& a, size_t idx, int i0,
 			else if (j == 0) ly = ld6(a.Min, idx + sy) - m;
 			else ly = ld6(a.Min, idx - sy) - m;
 		}
-		if (a.nz > 1) {
+		float ihz2 = a.ihz2;
+		if (a.nz > 1 && !(LAY && a.layered)) {
 			if (k > 0 && k < a.nz - 1) lz = ld6(a.Min, idx + sz) + ld6(a.Min, idx - sz) - 2.f * m;
 			else if (k == 0) lz = ld6(a.Min, idx + sz) - m;
 			else lz = ld6(a.Min, idx - sz) - m;
 		}
-		lap0 = a.ihx2 * lx0 + a.ihy2 * ly.a + a.ihz2 * lz.a;
-		lap1 = a.ihx2 * lx1 + a.ihy2 * ly.b + a.ihz2 * lz.b;
+		else if (LAY && a.lay_grouped && a.nz > 1) {
+			// planes of one 3D mesh in a stack, as in stage_cell
+			const int* grp = a.lay->grp;
+			const int g = grp[k];
+			const bool lo = k > 0 && grp[k - 1] == g, hi = k < a.nz - 1 && grp[k + 1] == g;
+			if (lo && hi) lz = ld6(a.Min, idx + sz) + ld6(a.Min, idx - sz) - 2.f * m;
+			else if (hi) lz = ld6(a.Min, idx + sz) - m;
+			else if (lo) lz = ld6(a.Min, idx - sz) - m;
+			ihz2 = a.lay->ihz2[k];
+		}
+		lap0 = a.ihx2 * lx0 + a.ihy2 * ly.a + ihz2 * lz.a;
+		lap1 = a.ihx2 * lx1 + a.ihy2 * ly.b + ihz2 * lz.b;
 	}
-	// the row kernel serves single meshes only (never a layer stack)
-	const CellMat cm{ a.A, a.alpha, a.K1 };
-	const F3 Ha{ a.Ha[0], a.Ha[1], a.Ha[2] };
+	const CellMat cm = LAY ? cell_mat(a, k) : CellMat{ a.A, a.alpha, a.K1 };
+	F3 Ha{ a.Ha[0], a.Ha[1], a.Ha[2] };
+	if (LAY && a.lay_field) Ha = F3{ a.lay->Ha[k][0], a.lay->Ha[k][1], a.lay->Ha[k][2] };
 	F3 H0 = eff_field(a, cm, Ha, m.a, Hd.a, lap0, Ms.x), H1 = eff_field(a, cm, Ha, m.b, Hd.b, lap1, Ms.y);
-	if (a.Hext) { const P6 he = ld6(a.Hext, idx); H0 = H0 + he.a; H1 = H1 + he.b; }
+	if (a.Hext) { const P6 he = LAY ? P6{ ld3(a.Hext, idx), ld3(a.Hext, idx + 1) } : ld6(a.Hext, idx); H0 = H0 + he.a; H1 = H1 + he.b; }
 	if (a.Heff_out) st6(a.Heff_out, idx, P6{ H0, H1 });
 	const P6 rhs{ llg_rhs(a, cm.alpha, m.a, H0, Ms.x), llg_rhs(a, cm.alpha, m.b, H1, Ms.y) };
 	return rk_update<METHOD, STEP>(a, idx, m, rhs, Ms, lte_loc);

@@ -74,3 +74,28 @@ def test_periodic_rows(gpu, n, pbc):
     ref = O.OracleDemag(n, H, pbc=pbc)(M0.astype(np.float64))
     assert rel(d.convolute(torch.from_numpy(M0).cuda()).cpu().numpy().astype(np.float64), ref) <= 1e-6
     d.close()
+
+
+@pytest.mark.parametrize("nx,ny,groups", [(64, 8, None), (128, 6, [0, 0, 1, 2, 2]), (192, 3, [0, 1, 1]), (512, 3, [0, 0])])
+@pytest.mark.parametrize("method", [api.BM_EVAL_RK4, api.BM_EVAL_RKDP54])
+def test_layer_stack_rows_match_the_separate_passes(gpu, monkeypatch, nx, ny, groups, method):
+    """Per-layer values, meshes of several planes, per-layer fields: the row kernel against the
+    separate x passes and stage kernel, the same arithmetic (FP32 rounding, 5 steps)."""
+    L = 3 if groups is None else len(groups)
+    rng = np.random.default_rng(nx)
+    p = api.FMParams(Ms=8e5, A=1.3e-11, alpha=0.1, K1=1e5, ea=(0.0, 0.0, 1.0), Ha=(1e4, 0.0, 2e4), modules=ALL)
+    M0 = (api.random_magnetisation(L * nx * ny, 1.0, 3) * 8e5).astype(np.float32)
+    out = []
+    for row in ("1", "0"):
+        monkeypatch.setenv("BM_ROW_KERNEL", row)
+        rng = np.random.default_rng(nx)
+        lay = dict(A=rng.uniform(1e-11, 2e-11, L), alpha=rng.uniform(0.02, 0.2, L), K1=rng.uniform(0, 2e5, L))
+        s = api.LayerStackSolver(method, nx, ny, 4e-9, 4e-9, [4e-9] * L, [4e-9 * l for l in range(L)], p, M0=M0, **lay)
+        s.set_layer_meshes(groups, rng.uniform(-2e4, 2e4, (L, 3)) if groups else None)
+        s.set_ms_map(np.repeat(rng.uniform(7e5, 9e5, L), nx * ny))
+        s.set_dt(2e-14)
+        s.set_astep(dT_max=2e-14)
+        s.run_to_iteration(5)
+        out.append(s.M.cpu().numpy().astype(np.float64))
+        s.close()
+    assert rel(out[0], out[1]) <= 5e-7
