@@ -337,12 +337,12 @@ int build_tables(bm_batch_s* o)
 			if (o->ml[b]) {
 				const MlView v = mlayer_view(o->ml[b]);
 				if (!col_ok(v.Ny, 0, v.L, v.NC, o->ncu)) continue;
-				Ny = v.Ny; kind = 0; t = ColBatch{ v.Sx, v.K, v.L, v.NC, v.NYH, v.ntl, v.ny };
+				Ny = v.Ny; kind = 0; t = ColBatch{ v.Sx, v.K, v.kcol, v.L, v.NC, v.NYH, v.ntl, v.ny };
 			}
 			else {
 				const bm_demag_s* d = o->dm[b];
 				if (!demag_col(d)) continue;
-				Ny = d->Ny; kind = d->Nz; full = d->full[1]; t = ColBatch{ d->Sx, d->K, d->nz, d->NC, d->NYH, d->ntl, full ? d->Ny : d->ny };
+				Ny = d->Ny; kind = d->Nz; full = d->full[1]; t = ColBatch{ d->Sx, d->K, nullptr, d->nz, d->NC, d->NYH, d->ntl, full ? d->Ny : d->ny };
 			}
 			col[(size_t)b] = 1;
 			bm_batch_s::ColGroup* g = nullptr;
@@ -511,7 +511,7 @@ int middle_all(bm_batch_s* o, hipStream_t st)
 	const std::vector<size_t> l2 = live(o->ty2), l4 = live(o->tyz[0]), l8 = live(o->tyz[1]), ly = live(o->ty), lz = live(o->tz), lm = live(o->tml);
 	const size_t nc = o->gcol.size();
 	int rc = fan(o, nc + l2.size() + l4.size() + l8.size(), st, [&](size_t q, hipStream_t s) {
-		if (q < nc) { auto& g = o->gcol[q]; return batch_col(g.Ny, g.kind, g.full, g.t.h.data(), g.t.d, (int)g.t.h.size(), s); }
+		if (q < nc) { auto& g = o->gcol[q]; return batch_col(g.Ny, g.kind, g.full, g.t.h.data(), g.t.d, (int)g.t.h.size(), o->ncu, s); }
 		if ((q -= nc) < l2.size()) {
 			const size_t g = l2[q];
 			return batch_y2d(o->gy2[g].size, o->gy2[g].full, o->gy2[g].sh[0], o->ty2[g].h.data(), o->ty2[g].d, (int)o->ty2[g].h.size(), o->ncu, s);

@@ -33,7 +33,33 @@ struct ColArgs {
 	float2* Sx; const float* K; const int* kidx;
 	int P, NC, NYH, ntl, nyd, lpk, tr;
 	const ColBatch* bt;     // batched: one mesh or stack per grid row
+	int ncu;                // compute units
 };
+
+// The columns kx = 0 and kx = N.x / 2 hold real values: in the z form from N.z = 16, whose
+// workgroups fill a compute unit each, the first workgroup takes both as one complex line (first + i second) where a column more
+// than a multiple of the compute units would cost a round of its own (RK4 steps: 256x256x8, 257
+// columns on 256 units, 235 -> 212 us, 256x128x16 242 -> 228, 512x256x8 389 -> 369).  A real line's transform is X(-ky) = conj X(ky), so the two spectra come apart
+// (and together) within the pair (ky, -ky): both are worked on for ky = 0 .. N.y / 2, column 0's
+// results at ky and the other's at N.y - ky, both in one value at ky = 0 and N.y / 2.
+__device__ __forceinline__ C2<float> pair_get(const C2<float>* line, int NY, int ky, int col)
+{
+	const C2<float> a = line[ky], b = line[ky ? NY - ky : 0];
+	return col ? mk(0.5f * (a.y + b.y), 0.5f * (b.x - a.x)) : mk(0.5f * (a.x + b.x), 0.5f * (a.y - b.y));
+}
+__device__ __forceinline__ void pair_put(C2<float>* line, int NY, int ky, int col, C2<float> w)
+{
+	if (ky == 0 || ky == NY / 2) { if (col) line[ky].y = w.x; else line[ky].x = w.x; }
+	else line[col ? NY - ky : ky] = w;
+}
+// the packed line's value at ky from what pair_put left
+__device__ __forceinline__ C2<float> pair_line(const C2<float>* line, int NY, int ky)
+{
+	const C2<float> v = line[ky];
+	if (ky == 0 || ky == NY / 2) return v;
+	const C2<float> o = line[NY - ky];
+	return ky < NY / 2 ? mk(v.x - o.y, v.y + o.x) : mk(o.x + v.y, v.x - o.y);
+}
 
 // the value of the lane whose number differs in bit 0 (or 1), within four lanes
 template <int CTRL> __device__ __forceinline__ C2<float> lane_quad(C2<float> v)
@@ -95,19 +121,22 @@ template <int NZ> struct ZLanes {
 	}
 };
 
-template <int NY, int KIND, int NZ, bool FULL>
-__global__ void __launch_bounds__((col_threads<KIND, NZ>())) k_col(ColArgs a)
+__device__ __host__ __forceinline__ bool col_packed(int lpk, int NC, int ncu) { return lpk == 1 && NC > ncu && (NC - 1) % ncu == 0; }
+
+template <int NY, int KIND, int NZ, bool FULL, bool PACK>
+__global__ void __launch_bounds__((col_threads<KIND, NZ>()), (KIND == COL_LAYERS && NY < 1024 ? 4 : 1)) k_col(ColArgs a)
 {
 	constexpr int E = Plan<NY>::E, T = plan_T<NY>(), LW = 64 / T, LL = lds_len<NY>(), EL = FULL ? E : E / 2, NZH = NZ / 2 + 1;
 	static_assert(T <= 64, "a line must lie within one wave");
 	extern __shared__ C2<float> lb[];
 	if (a.bt) {
 		const ColBatch& b = a.bt[blockIdx.y];
-		a.Sx = b.Sx; a.K = b.K; a.P = b.P; a.NC = b.NC; a.NYH = b.NYH; a.ntl = b.ntl; a.nyd = b.nyd;
-		if ((int)blockIdx.x * a.lpk >= a.NC) return;          // uniform over the block
+		a.Sx = b.Sx; a.K = b.K; a.kidx = b.kidx; a.P = b.P; a.NC = b.NC; a.NYH = b.NYH; a.ntl = b.ntl; a.nyd = b.nyd;
 	}
 	const int lane = threadIdx.x & 63, t = lane % T, sub = lane / T, stride = (blockDim.x >> 6) * LW;
 	const int P = KIND == COL_2D ? 1 : a.P, lpk = a.lpk, nl = 3 * P * lpk, kx0 = blockIdx.x * lpk;
+	const bool packed = PACK && col_packed(lpk, a.NC, a.ncu), both = PACK && packed && blockIdx.x == 0;
+	if (kx0 >= a.NC - (packed ? 1 : 0)) return;                 // uniform over the block
 	Twiddles<NY, float> tw; tw.init(t);
 
 	// lines li = (c P + z) lpk + column: the next round's values are loaded while this one's are
@@ -120,7 +149,10 @@ __global__ void __launch_bounds__((col_threads<KIND, NZ>())) k_col(ColArgs a)
 		for (int e = 0; e < EL; e++) {
 			const int y = t + T * e;
 			float2 q = make_float2(0.f, 0.f);
-			if (ok && y < a.nyd) q = a.Sx[sx_line(cz, kx, y, a.NC, a.ntl)];
+			if (ok && y < a.nyd) {
+				q = a.Sx[sx_line(cz, kx, y, a.NC, a.ntl)];
+				if (both) q.y = a.Sx[sx_line(cz, a.NC - 1, y, a.NC, a.ntl)].x;
+			}
 			pre[e] = mk(q.x, q.y);
 		}
 	};
@@ -156,7 +188,8 @@ __global__ void __launch_bounds__((col_threads<KIND, NZ>())) k_col(ColArgs a)
 		}
 	}
 	else if constexpr (KIND == COL_LAYERS) {
-		// item (destination d, column, ky); own layer first, then the others in order (k_ml_mult)
+		// item (destination d, column, ky); own layer first, then the others in order (k_ml_mult); four
+		// sources' kernel loads in flight (ten 128x64 layers: 32.4 -> 27.0 us with the shared kernels)
 		const size_t kq = (size_t)a.NC * a.NYH;
 		const int items = P * lpk * NY, cs = P * lpk * LL;        // component stride of the lines
 		const float tz = a.tr ? -1.f : 1.f;
@@ -171,6 +204,7 @@ __global__ void __launch_bounds__((col_threads<KIND, NZ>())) k_col(ColArgs a)
 				const float sy = up ? -1.f : 1.f;
 				const float* Kb = a.K + (size_t)kx * a.NYH + (up ? NY - ky : ky);
 				const C2<float>* Fb = lb + il * LL + ky;
+#pragma unroll 4
 				for (int r = 0; r < P; r++) {
 					const int s = r == 0 ? d : (r <= d ? r - 1 : r), p = a.tr ? s * P + d : d * P + s;
 					const float* Kp = Kb + (size_t)(a.kidx ? a.kidx[p] : p) * 6 * kq;
@@ -190,8 +224,7 @@ __global__ void __launch_bounds__((col_threads<KIND, NZ>())) k_col(ColArgs a)
 		for (int n = 0; n < kColItems; n++) {
 			const int i = threadIdx.x + n * blockDim.x;
 			if (i < items) {
-				const int ky = i % NY, dl = i / NY;
-				C2<float>* p = lb + dl * LL + ky;                 // dl = d lpk + column, as the lines are
+				C2<float>* p = lb + (i / NY) * LL + i % NY;       // i / NY = d lpk + column, as the lines are
 #pragma unroll
 				for (int c = 0; c < 3; c++) p[c * cs] = mk(o[n][c].x, o[n][c].y);
 			}
@@ -203,17 +236,21 @@ __global__ void __launch_bounds__((col_threads<KIND, NZ>())) k_col(ColArgs a)
 		const size_t kq = (size_t)a.NC * a.NYH * NZH;
 		const int zs = lpk * LL, cs = P * zs, zt = threadIdx.x % M;
 		Twiddles<NZ, float> tz; tz.init(zt);
-		for (int i = threadIdx.x; i < lpk * NY * M; i += blockDim.x) {
-			const int j = i / M, il = j / NY, ky = j % NY, kx = min(kx0 + il, a.NC - 1);
+		// both: the pair's two items run in adjacent lanes and read before either writes
+		for (int i = threadIdx.x; i < (both ? NY + 2 : lpk * NY) * M; i += blockDim.x) {
+			const int j = i / M, il = both ? 0 : j / NY, col = both ? j & 1 : 0, ky = both ? j >> 1 : j % NY;
+			const int kx = col ? a.NC - 1 : min(kx0 + il, a.NC - 1);
 			const int kyr = ky <= NY / 2 ? ky : NY - ky;
 			const float sy = ky <= NY / 2 ? 1.f : -1.f;
 			const float* kb = a.K + ((size_t)kx * a.NYH + kyr) * NZH;
-			C2<float>* p = lb + il * LL + ky;
+			C2<float>* p = lb + il * LL;
 			C2<float> u[3][NF];
 #pragma unroll
 			for (int c = 0; c < 3; c++) {
 #pragma unroll
-				for (int e = 0; e < NF; e++) { const int z = zt + M * e; u[c][e] = M * e < ZD && z < P ? p[c * cs + z * zs] : mk(0.f, 0.f); }
+				for (int e = 0; e < NF; e++) { const int z = zt + M * e; 
+					u[c][e] = M * e < ZD && z < P ? (both ? pair_get(p + c * cs + z * zs, NY, ky, col) : p[c * cs + z * zs + ky]) : mk(0.f, 0.f);
+				}
 				ZLanes<NZ>::template run<-1>(u[c], zt, tz);
 			}
 #pragma unroll
@@ -231,7 +268,13 @@ __global__ void __launch_bounds__((col_threads<KIND, NZ>())) k_col(ColArgs a)
 			for (int c = 0; c < 3; c++) {
 				ZLanes<NZ>::template run<1>(u[c], zt, tz);
 #pragma unroll
-				for (int e = 0; e < NF; e++) { const int z = zt + M * e; if (M * e < ZD && z < P) p[c * cs + z * zs] = u[c][e]; }
+				for (int e = 0; e < NF; e++) {
+					const int z = zt + M * e;
+					if (M * e < ZD && z < P) {
+						if (both) pair_put(p + c * cs + z * zs, NY, ky, col, u[c][e]);
+						else p[c * cs + z * zs + ky] = u[c][e];
+					}
+				}
 			}
 		}
 	}
@@ -242,14 +285,16 @@ __global__ void __launch_bounds__((col_threads<KIND, NZ>())) k_col(ColArgs a)
 		C2<float>* line = lb + li * LL;
 		C2<float> v[E];
 #pragma unroll
-		for (int e = 0; e < E; e++) v[e] = line[t + T * e];
+		for (int e = 0; e < E; e++) v[e] = both ? pair_line(line, NY, t + T * e) : line[t + T * e];
 		xsync<true>();
 		fft<NY, 1, float, true>(v, line, 1, t, tw);
 		if (li < nl && kx < a.NC) {
 #pragma unroll
 			for (int e = 0; e < EL; e++) {
 				const int y = t + T * e;
-				if (y < a.nyd) a.Sx[sx_line(cz, kx, y, a.NC, a.ntl)] = make_float2(v[e].x, v[e].y);
+				if (y >= a.nyd) continue;
+				a.Sx[sx_line(cz, kx, y, a.NC, a.ntl)] = make_float2(v[e].x, both ? 0.f : v[e].y);
+				if (both) a.Sx[sx_line(cz, a.NC - 1, y, a.NC, a.ntl)] = make_float2(v[e].y, 0.f);
 			}
 		}
 	}
@@ -263,22 +308,27 @@ template <int NY, int KIND, int NZ> ColShape col_shape(int P)
 	ColShape s;
 	s.lpk = std::max(1, 64 / (3 * P * T));
 	const int nl = 3 * P * s.lpk, nlp = (nl + LW - 1) / LW * LW;
-	// a wave per LW lines; more for the layers form where its items need them
-	const int waves = std::max(nlp / LW, KIND == COL_LAYERS ? (P * s.lpk * NY + 64 * kColItems - 1) / (64 * kColItems) : 0);
+	// a wave per LW lines; more where the product's items need them
+	int waves = nlp / LW;
+	if constexpr (KIND == COL_LAYERS) waves = std::max(waves, (P * s.lpk * NY + 64 * kColItems - 1) / (64 * kColItems));
+	if constexpr (KIND == COL_Z) waves = std::max(waves, (s.lpk * NY * plan_T<NZ>() + 63) / 64);
 	s.threads = std::min(col_threads<KIND, NZ>(), 64 * waves);
 	s.lds = (size_t)nlp * LL * sizeof(C2<float>);
 	return s;
 }
 
-template <int NY, int KIND, int NZ, bool FULL>
+template <int NY, int KIND, int NZ, bool FULL, bool PACK = false>
 int launch_col_t(const ColArgs& in, int nb, hipStream_t st)
 {
+	// the z form with one workgroup per compute unit: columns 0 and N.x / 2 as one
+	if constexpr (KIND == COL_Z && NZ >= 16 && !PACK)
+		if (in.bt ? in.NC > in.ncu : col_packed(col_shape<NY, KIND, NZ>(in.P).lpk, in.NC, in.ncu)) return launch_col_t<NY, KIND, NZ, FULL, true>(in, nb, st);
 	const ColShape s = col_shape<NY, KIND, NZ>(in.P);
 	ColArgs a = in;
 	a.lpk = s.lpk;
 	if (s.lds > 65536)
-		BM_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(&k_col<NY, KIND, NZ, FULL>), hipFuncAttributeMaxDynamicSharedMemorySize, (int)s.lds));
-	hipLaunchKernelGGL((k_col<NY, KIND, NZ, FULL>), dim3((a.NC + s.lpk - 1) / s.lpk, nb), dim3(s.threads), s.lds, st, a);
+		BM_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(&k_col<NY, KIND, NZ, FULL, PACK>), hipFuncAttributeMaxDynamicSharedMemorySize, (int)s.lds));
+	hipLaunchKernelGGL((k_col<NY, KIND, NZ, FULL, PACK>), dim3((a.NC - (PACK && !a.bt) + s.lpk - 1) / s.lpk, nb), dim3(s.threads), s.lds, st, a);
 	return BM_OK;
 }
 
@@ -309,7 +359,7 @@ bool bm::col_ok(int Ny, int kind, int P, int NC, int ncu)
 	if (kind >= 16 && Ny % 3 == 0 && NC > ncu) return false;
 	switch (Ny) {
 #define C_(V_) case V_: { if (!kind) return col_items<V_, 1>(P) || col_items<V_, 2>(P); \
-		return col_shape<V_, COL_Z, 1>(P).lds <= kColLds; }
+		return col_shape<V_, COL_Z, 4>(P).lds <= kColLds; }
 	BM_FOR_COL_SIZES(C_)
 #undef C_
 	}
@@ -336,16 +386,17 @@ int launch_any(int Ny, int kind, bool full, const ColArgs& a, int nb, hipStream_
 }
 }
 
-int bm::launch_col(int Ny, int kind, bool full, float2* Sx, const float* K, const int* kidx, int P, int NC, int NYH, int ntl, int nyd, int tr, hipStream_t st)
+int bm::launch_col(int Ny, int kind, bool full, float2* Sx, const float* K, const int* kidx, int P, int NC, int NYH, int ntl, int nyd, int tr, int ncu,
+	hipStream_t st)
 {
-	return launch_any(Ny, kind, full, ColArgs{ Sx, K, kidx, P, NC, NYH, ntl, nyd, 1, tr, nullptr }, 1, st);
+	return launch_any(Ny, kind, full, ColArgs{ Sx, K, kidx, P, NC, NYH, ntl, nyd, 1, tr, nullptr, ncu }, 1, st);
 }
 
 // sized by the largest mesh: LDS and threads by its planes, grid rows by its columns
-int bm::batch_col(int Ny, int kind, bool full, const ColBatch* h_tab, const ColBatch* d_tab, int nb, hipStream_t st)
+int bm::batch_col(int Ny, int kind, bool full, const ColBatch* h_tab, const ColBatch* d_tab, int nb, int ncu, hipStream_t st)
 {
 	ColArgs a{};
-	a.lpk = 1; a.bt = d_tab;
+	a.lpk = 1; a.bt = d_tab; a.ncu = ncu;
 	for (int b = 0; b < nb; b++) { a.P = std::max(a.P, h_tab[b].P); a.NC = std::max(a.NC, h_tab[b].NC); }
 	return launch_any(Ny, kind, full, a, nb, st);
 }

@@ -124,10 +124,11 @@ int batch_inv_xs_planar(int HX, bool full, const struct PassBatch* h_tab, const 
 // The middle passes as one kernel per kx column group (bm_col.hip): whether it serves N.y, kind (N.z
 // of a 3D mesh, 1: 2D, 0: layers), P planes or layers and NC columns, and its launcher (full:
 // periodic y; tr: the layers' transposed product).
-struct ColBatch { float2* Sx; const float* K; int P, NC, NYH, ntl, nyd; };   // one mesh or stack of a batched launch
+struct ColBatch { float2* Sx; const float* K; const int* kidx; int P, NC, NYH, ntl, nyd; };   // one mesh or stack of a batched launch
 bool col_ok(int Ny, int kind, int P, int NC, int ncu);
-int batch_col(int Ny, int kind, bool full, const ColBatch* h_tab, const ColBatch* d_tab, int nb, hipStream_t st);
-int launch_col(int Ny, int kind, bool full, float2* Sx, const float* K, const int* kidx, int P, int NC, int NYH, int ntl, int nyd, int tr, hipStream_t st);
+int batch_col(int Ny, int kind, bool full, const ColBatch* h_tab, const ColBatch* d_tab, int nb, int ncu, hipStream_t st);
+int launch_col(int Ny, int kind, bool full, float2* Sx, const float* K, const int* kidx, int P, int NC, int NYH, int ntl, int nyd, int tr, int ncu,
+	hipStream_t st);
 // Per-mesh arguments of the other passes in a batched launch (the fields each pass uses;
 // the y passes take ny as the data rows of a line).
 struct PassBatch {
@@ -156,7 +157,7 @@ bool plan_2d_pbc_ok(int nx, int ny, bool fx, bool fy);
 void mlayer_pbc(const bm_mlayer_s* m, int out[2]);
 // Pointers and sizes of a multilayered demag handle (batched launches).
 struct MlView {
-	float2* Sx; float2* S; const float* K;
+	float2* Sx; float2* S; const float* K; const int* kcol;
 	int L, nx, ny, Nx, Ny, NC, NYH, Sp, ntl;
 };
 MlView mlayer_view(bm_mlayer_s* m);

@@ -572,6 +572,8 @@ struct bm_mlayer_s {
 	int nslot = 0;
 	std::vector<int> hkidx;  // slot of pair (d, s) at d * L + s
 	int* kidx = nullptr;     // its device copy (L > kRegLayers)
+	int* kcol = nullptr;     // column pass: the kernel each pair reads, the first pair's of its slot where
+	                         // every pair holds a copy (so that equal pairs share cache lines)
 	bool per_pair() const { return L <= kRegLayers; }
 	size_t kbase(int d, int s) const { return (size_t)(per_pair() ? d * L + s : hkidx[(size_t)d * L + s]); }
 	long long kcount = 0, bytes = 0;
@@ -863,12 +865,17 @@ static int ml_create_grid(int nlayers, int nx, int ny, double hx, double hy, con
 		|| (ncx && hipMalloc(&m->Kc, (size_t)ncx * 12 * m->NC * m->Ny * sizeof(float)) != hipSuccess)
 		|| (ncx && hipMalloc(&m->kcoff, m->hkcoff.size() * sizeof(long long)) != hipSuccess)
 		|| hipMalloc(&m->K, (size_t)m->kcount * sizeof(float)) != hipSuccess
+		|| hipMalloc(&m->kcol, m->hkidx.size() * sizeof(int)) != hipSuccess
 		|| (nlayers > kRegLayers && hipMalloc(&m->kidx, m->hkidx.size() * sizeof(int)) != hipSuccess)
 		|| hipMalloc(&m->ebuf, (size_t)bm::x_plane_parts(m->xs, ny) * sizeof(double)) != hipSuccess) {
 		bm_mlayer_destroy(m);
 		return fail(BM_ERR_NOMEM, "bm_mlayer_create: device memory");
 	}
-	if ((m->kidx && hipMemcpy(m->kidx, m->hkidx.data(), m->hkidx.size() * sizeof(int), hipMemcpyHostToDevice) != hipSuccess)
+	std::vector<int> kcol(m->hkidx);
+	if (m->per_pair())
+		for (size_t pr = 0; pr < kcol.size(); pr++) kcol[pr] = (int)(std::find(m->hkidx.begin(), m->hkidx.end(), m->hkidx[pr]) - m->hkidx.begin());
+	if (hipMemcpy(m->kcol, kcol.data(), kcol.size() * sizeof(int), hipMemcpyHostToDevice) != hipSuccess
+		|| (m->kidx && hipMemcpy(m->kidx, m->hkidx.data(), m->hkidx.size() * sizeof(int), hipMemcpyHostToDevice) != hipSuccess)
 		|| (m->kcoff && hipMemcpy(m->kcoff, m->hkcoff.data(), m->hkcoff.size() * sizeof(long long), hipMemcpyHostToDevice) != hipSuccess)) {
 		bm_mlayer_destroy(m);
 		return fail(BM_ERR_HIP, "bm_mlayer_create: pair table");
@@ -1125,6 +1132,7 @@ extern "C" int bm_mlayer_destroy(bm_mlayer_t m)
 	if (m->Kc) (void)hipFree(m->Kc);
 	if (m->kcoff) (void)hipFree(m->kcoff);
 	if (m->kidx) (void)hipFree(m->kidx);
+	if (m->kcol) (void)hipFree(m->kcol);
 	if (m->ebuf) (void)hipFree(m->ebuf);
 	if (m->tabs) (void)hipFree(m->tabs);
 	if (m->stage) (void)hipFree(m->stage);
@@ -1146,7 +1154,7 @@ int bm::mlayer_mid(bm_mlayer_s* m, hipStream_t st, int tr)
 	if (!m->Kc && bm::col_ok(m->Ny, 0, L, m->NC, m->ncu)) {
 		// the y passes and the product as one, timed as the product
 		bm::prof_mark_begin(bm::PK_ML_MULT, st);
-		rc = bm::launch_col(m->Ny, 0, fy, m->Sx, m->K, m->kidx, L, m->NC, m->NYH, m->ntl, fy ? m->Ny : m->ny, tr, st);
+		rc = bm::launch_col(m->Ny, 0, fy, m->Sx, m->K, m->kcol, L, m->NC, m->NYH, m->ntl, fy ? m->Ny : m->ny, tr, m->ncu, st);
 		bm::prof_mark_end(bm::PK_ML_MULT, st);
 		return rc;
 	}
@@ -1183,7 +1191,7 @@ double bm::mlayer_z0(const bm_mlayer_s* m, int l) { return m->z0[(size_t)l]; }
 
 bm::MlView bm::mlayer_view(bm_mlayer_s* m)
 {
-	return MlView{ m->Sx, m->S, m->K, m->L, m->nx, m->ny, m->Nx, m->Ny, m->NC, m->NYH, m->Sp, m->ntl };
+	return MlView{ m->Sx, m->S, m->K, m->kcol, m->L, m->nx, m->ny, m->Nx, m->Ny, m->NC, m->NYH, m->Sp, m->ntl };
 }
 
 int bm::batch_ml_mult(int L, LaunchShape sh, const MlBatch* h_tab, const MlBatch* d_tab, int nb, int ncu, hipStream_t st)

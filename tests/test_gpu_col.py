@@ -66,3 +66,23 @@ def test_layers(gpu, nx, ny, L, pbc):
     ref = O.OracleMLayer(nx, ny, 4e-9, 4e-9, np.array(hz), np.array(z0), pbc)(M0.astype(np.float64))
     assert rel(d.convolute(torch.from_numpy(M0).cuda()).cpu().numpy().astype(np.float64), np.asarray(ref).reshape(-1, 3)) <= 1e-6
     d.close()
+
+
+@pytest.mark.parametrize("n", [(256, 64, 1), (256, 33, 8), (256, 24, 3), (512, 32, 2), (512, 128, 12), (256, 96, 6), (512, 100, 1)])
+def test_first_and_last_column_as_one(gpu, n):
+    """N.x / 2 a multiple of the compute units: columns 0 and N.x / 2 share a workgroup."""
+    M0 = api.random_magnetisation(n[0] * n[1] * n[2], 8e5, 2).astype(np.float32)
+    d = api.Demag(n, H)
+    ref = O.OracleDemag(n, H, Nz_override=nz_open(n[2]))(M0.astype(np.float64))
+    assert rel(d.convolute(torch.from_numpy(M0).cuda()).cpu().numpy().astype(np.float64), ref) <= 1e-6
+    d.close()
+
+
+@pytest.mark.parametrize("nx,ny,L", [(256, 32, 3), (256, 64, 6), (512, 24, 4)])
+def test_layers_first_and_last_column_as_one(gpu, nx, ny, L):
+    z0 = [8e-9 * l for l in range(L)]
+    M0 = api.random_magnetisation(nx * ny * L, 8e5, 6).astype(np.float32)
+    d = api.MultiLayerDemag(nx, ny, 4e-9, 4e-9, [4e-9] * L, z0)
+    ref = O.OracleMLayer(nx, ny, 4e-9, 4e-9, np.full(L, 4e-9), np.array(z0))(M0.astype(np.float64))
+    assert rel(d.convolute(torch.from_numpy(M0).cuda()).cpu().numpy().astype(np.float64), np.asarray(ref).reshape(-1, 3)) <= 1e-6
+    d.close()
