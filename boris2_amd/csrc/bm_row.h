@@ -243,7 +243,7 @@ int launch_row_t(const RowGeom& d, const StageArgs& a, float scale, hipStream_t 
 #define C_(V_) case V_: { \
 	if constexpr (xs_ok<V_>()) if (xs_few_rows(V_, d.ny, d.nz, d.ncu, true)) { \
 		const int ns = (d.ny + XSplit<V_>::RP - 1) / XSplit<V_>::RP, g = d.nz * ns; \
-		const dim3 gd((g + 7) / 8 * 8), bd(XSplit<V_>::BS); \
+		const dim3 gd((g + 7) / 8 * 8), bd(a.layered ? XSplit<V_, xs_groups<V_, true>()>::BS : XSplit<V_, xs_groups<V_>()>::BS); \
 		if (a.layered) hipLaunchKernelGGL((k_rows<V_, METHOD, STEP, R2C, true>), gd, bd, 0, st, a, d.Sx, d.ntl, ns, scale); \
 		else hipLaunchKernelGGL((k_rows<V_, METHOD, STEP, R2C, false>), gd, bd, 0, st, a, d.Sx, d.ntl, ns, scale); \
 		return BM_OK; \

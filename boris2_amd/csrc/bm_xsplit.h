@@ -28,11 +28,23 @@ template <int HX> constexpr bool xs_ok() { return plan_T<HX>() <= 64; }
 // lengths whose row kernel always takes this form (see xs_few_rows)
 template <int HX> constexpr bool xs_row_only() { return xs_ok<HX>() && Plan<HX>::E == 12; }
 
-template <int HX> struct XSplit {
-	static constexpr int W = xs_waves<HX>(), WT = 64 * W, BS = 3 * WT, E = Plan<HX>::E, T = plan_T<HX>();
+// wave groups of the kernels with much per-cell work: with 8 values per thread the 32 W E cell pairs of
+// a workgroup are a third more than three groups, so rows of 16 lanes or fewer take a fourth wave for
+// the per-cell work only (one round instead of two: 128x64 film RK4 step 48.1 -> 46.9 us, ten 128x64
+// layers 105 -> 101).  At 256 cells per row (32 lanes) it pays for layer stacks, which are small (LAY;
+// RK4 step of three 256x256 layers 116 -> 111 us), and costs larger meshes more (256x256x8, three
+// RKDP54 steps 1024 -> 1064 us).
+template <int HX, bool LAY = false> constexpr int xs_groups()
+{
+	return xs_waves<HX>() == 1 && Plan<HX>::E == 8 && plan_T<HX>() <= (LAY ? 32 : 16) ? 4 : 3;
+}
+
+template <int HX, int NG = 3> struct XSplit {
+	static constexpr int W = xs_waves<HX>(), WT = 64 * W, E = Plan<HX>::E, T = plan_T<HX>();
+	static constexpr int BS = NG * WT;
 	static constexpr int RP = WT / T, NC = HX + 1, P = xrow_pitch<HX>();
 	static constexpr int NL = (RP * NC + WT - 1) / WT;   // spectra values per thread of one component
-	int c, q;                // component, thread within its wave group
+	int c, q;                // component (3: the fourth wave), thread within its wave group
 	C2<float>* mine;         // this component's rows
 	C2<float>* row;          // this thread's row
 	XThread<HX> th;
@@ -49,6 +61,7 @@ template <int HX> struct XSplit {
 
 	__device__ __forceinline__ void load(const float2* Sx, int z, int y0, int ny, int nzs, int ntl) const
 	{
+		if (c > 2) return;
 		const float2* base = Sx + sx_base(c, z, y0, nzs, NC, ntl);
 		float2 r[NL];
 #pragma unroll
@@ -68,6 +81,7 @@ template <int HX> struct XSplit {
 	}
 	__device__ __forceinline__ void store(float2* Sx, int z, int y0, int ny, int nzs, int ntl) const
 	{
+		if (c > 2) return;
 		float2* base = Sx + sx_base(c, z, y0, nzs, NC, ntl);
 #pragma unroll
 		for (int l = 0; l < NL; l++) {
@@ -80,6 +94,7 @@ template <int HX> struct XSplit {
 	// this thread's row from the spectra in LDS to EL scaled cell pairs in LDS (pair k at k)
 	template <int EL> __device__ __forceinline__ void c2r(float scale)
 	{
+		if (c > 2) return;
 		C2<float> v[E];
 		c2r_row<HX, true>(th, row, v);
 		xsync<true>();                   // the transform's last LDS reads are done
@@ -89,6 +104,7 @@ template <int HX> struct XSplit {
 	// the reverse: EL cell pairs in LDS (zero above) to the row's spectra in LDS
 	template <int EL> __device__ __forceinline__ void r2c()
 	{
+		if (c > 2) return;
 		C2<float> v[E];
 #pragma unroll
 		for (int e = 0; e < E; e++) v[e] = e < EL ? row[th.t + T * e] : mk(0.f, 0.f);
@@ -140,12 +156,13 @@ __global__ void __launch_bounds__(XSplit<HX>::BS) k_fwd_xs(FwdArgs a, const FwdA
 
 // P5 (k_inv_x) in this form; modes as there.  The interleaved outputs go through LDS so that a
 // thread moves whole cell pairs.
+template <int HX, int MODE> constexpr int xs_inv_groups() { return MODE == 0 ? 3 : xs_groups<HX>(); }
 template <int HX, int MODE, bool EN, bool FULL, bool GEN>
-__global__ void __launch_bounds__(XSplit<HX>::BS) k_inv_xs(const float2* __restrict__ Sx, float* __restrict__ out,
+__global__ void __launch_bounds__((XSplit<HX, xs_inv_groups<HX, MODE>()>::BS)) k_inv_xs(const float2* __restrict__ Sx, float* __restrict__ out,
 	int ny, int nz, int ntl, float scale, const float* __restrict__ M, double* __restrict__ epart,
 	int nxr, int zoff, int nzl, const PassBatch* __restrict__ bt)
 {
-	using X = XSplit<HX>;
+	using X = XSplit<HX, xs_inv_groups<HX, MODE>()>;
 	if (bt) { const PassBatch& b = bt[blockIdx.y]; Sx = b.Sx; out = b.out; ny = b.ny; nz = b.nz; ntl = b.ntl; scale = b.scale; }
 	__shared__ C2<float> tile[3 * X::RP * X::P];
 	__shared__ double ered[EN ? X::BS : 1];
@@ -162,7 +179,7 @@ __global__ void __launch_bounds__(XSplit<HX>::BS) k_inv_xs(const float2* __restr
 		double esum = 0.0;
 		if constexpr (MODE == 0) {
 			// planar: each wave group stores its own component
-			for (int p = x.q; p < X::RP * NP; p += X::WT) {
+			for (int p = x.q; x.c < 3 && p < X::RP * NP; p += X::WT) {
 				const int r = p / NP, k = p % NP, y = y0 + r;
 				if (y >= ny) continue;
 				const C2<float> h = x.mine[r * X::P + k];
@@ -211,9 +228,9 @@ __global__ void __launch_bounds__(XSplit<HX>::BS) k_inv_xs(const float2* __restr
 // The fused row kernel (k_row) in this form; LAY: a layer stack (the planes are the layers), a form of
 // its own because the per-layer values cost plain meshes 3 % (RK4 step of a 128x64 film 47.8 -> 49.5 us).
 template <int HX, int METHOD, int STEP, bool R2C, bool LAY>
-__global__ void __launch_bounds__(XSplit<HX>::BS) k_rows(StageArgs a, float2* Sx, int ntl, int ntiles, float scale)
+__global__ void __launch_bounds__((XSplit<HX, xs_groups<HX, LAY>()>::BS)) k_rows(StageArgs a, float2* Sx, int ntl, int ntiles, float scale)
 {
-	using X = XSplit<HX>;
+	using X = XSplit<HX, xs_groups<HX, LAY>()>;
 	__shared__ C2<float> tile[3 * X::RP * X::P];
 	X x; x.init(tile);
 	constexpr int EL = X::E / 2, NP = HX / 2;

@@ -12,8 +12,8 @@ void inv_var(int mode, dim3 g, hipStream_t st, const float2* Sx, float* out, int
 	const float* M, double* epart, int nx, int zoff, int nzl)
 {
 	const PassBatch* nb = nullptr;
-	const dim3 b(XSplit<HX>::BS);
-	if (mode == 0) hipLaunchKernelGGL((k_inv_xs<HX, 0, false, FULL, GEN>), g, b, 0, st, Sx, out, ny, nz, ntl, scale, M, epart, nx, zoff, nzl, nb);
+	const dim3 b(XSplit<HX, xs_groups<HX>()>::BS);
+	if (mode == 0) hipLaunchKernelGGL((k_inv_xs<HX, 0, false, FULL, GEN>), g, dim3(XSplit<HX>::BS), 0, st, Sx, out, ny, nz, ntl, scale, M, epart, nx, zoff, nzl, nb);
 	else if (mode == 1 && !epart) hipLaunchKernelGGL((k_inv_xs<HX, 1, false, FULL, GEN>), g, b, 0, st, Sx, out, ny, nz, ntl, scale, M, epart, nx, zoff, nzl, nb);
 	else if (mode == 1) hipLaunchKernelGGL((k_inv_xs<HX, 1, true, FULL, GEN>), g, b, 0, st, Sx, out, ny, nz, ntl, scale, M, epart, nx, zoff, nzl, nb);
 	else if (!epart) hipLaunchKernelGGL((k_inv_xs<HX, 2, false, FULL, GEN>), g, b, 0, st, Sx, out, ny, nz, ntl, scale, M, epart, nx, zoff, nzl, nb);
