@@ -24,6 +24,7 @@
 // forward 4 convolutions per step; backward 4 (recompute) + 4 (adjoint) per step.
 #include "bm_internal.h"
 #include "bm_stage.h"
+#include "bm_adjcell.h"
 
 #include <algorithm>
 #include <cmath>
@@ -32,92 +33,9 @@
 
 using namespace bm;
 
-// layer stacks in the adjoint: per-layer values passed in the kernel arguments (8 layers)
-constexpr int kMaxAdjLayers = 8;
-
 namespace {
 
 constexpr int kAB = 256;
-
-struct AdjArgs {
-	int nx, ny, nz;
-	float ihx2, ihy2, ihz2;
-	float A, alpha, grel;
-	float K1, K2, ea[3];    // uniaxial anisotropy
-	float Hz[3];            // applied field at the step's start time
-	float dir[3], sc;       // pulse direction and sinc value at that time (d H / d amp = sc dir)
-	float tz;               // ramp: d H / d slope_c = tz e_c (the step's start time), else 0
-	int modules;
-	const float* Ms;
-	int layered;            // layer stack: per-layer A, alpha, K1, no exchange across layers
-	int per;                // periodic exchange along x, y, z: bits 0, 1, 2
-	float lay_A[kMaxAdjLayers], lay_alpha[kMaxAdjLayers], lay_K1[kMaxAdjLayers];
-};
-
-__device__ __forceinline__ CellMat adj_mat(const AdjArgs& a, int k)
-{
-	if (!a.layered) return CellMat{ a.A, a.alpha, a.K1 };
-	CellMat c{ a.lay_A[0], a.lay_alpha[0], a.lay_K1[0] };
-#pragma unroll
-	for (int l = 1; l < kMaxAdjLayers; l++)
-		if (k == l) c = CellMat{ a.lay_A[l], a.lay_alpha[l], a.lay_K1[l] };
-	return c;
-}
-
-__device__ __forceinline__ F3 lap_at(const float* X, const AdjArgs& a, size_t idx, int i, int j, int k)
-{
-	const F3 m = ld3(X, idx);
-	F3 lx{ 0, 0, 0 }, ly{ 0, 0, 0 }, lz{ 0, 0, 0 };
-	const size_t sy = a.nx, sz = (size_t)a.nx * a.ny;
-	// periodic axes at the mesh ends: the wrapped neighbour (BorisLib/VEC_VC_Del.h:24-45)
-	if (a.nx > 1) {
-		if (i > 0 && i < a.nx - 1) lx = ld3(X, idx + 1) + ld3(X, idx - 1) - 2.f * m;
-		else if (a.per & 1) lx = (i == 0) ? ld3(X, idx + 1) + ld3(X, idx + (a.nx - 1)) - 2.f * m
-		                                  : ld3(X, idx - (a.nx - 1)) + ld3(X, idx - 1) - 2.f * m;
-		else if (i == 0) lx = ld3(X, idx + 1) - m;
-		else lx = ld3(X, idx - 1) - m;
-	}
-	if (a.ny > 1) {
-		if (j > 0 && j < a.ny - 1) ly = ld3(X, idx + sy) + ld3(X, idx - sy) - 2.f * m;
-		else if (a.per & 2) ly = (j == 0) ? ld3(X, idx + sy) + ld3(X, idx + (a.ny - 1) * sy) - 2.f * m
-		                                  : ld3(X, idx - (a.ny - 1) * sy) + ld3(X, idx - sy) - 2.f * m;
-		else if (j == 0) ly = ld3(X, idx + sy) - m;
-		else ly = ld3(X, idx - sy) - m;
-	}
-	if (a.nz > 1 && !a.layered) {
-		if (k > 0 && k < a.nz - 1) lz = ld3(X, idx + sz) + ld3(X, idx - sz) - 2.f * m;
-		else if (a.per & 4) lz = (k == 0) ? ld3(X, idx + sz) + ld3(X, idx + (a.nz - 1) * sz) - 2.f * m
-		                                  : ld3(X, idx - (a.nz - 1) * sz) + ld3(X, idx - sz) - 2.f * m;
-		else if (k == 0) lz = ld3(X, idx + sz) - m;
-		else lz = ld3(X, idx - sz) - m;
-	}
-	return a.ihx2 * lx + a.ihy2 * ly + a.ihz2 * lz;
-}
-
-__device__ __forceinline__ float cex(float A, float Ms) { return (2.f * A) / ((float)kMU0 * Ms * Ms); }
-__device__ __forceinline__ float pre_llg(const AdjArgs& a, float alpha) { return (float)(-kGAMMA) * a.grel / (1.f + alpha * alpha); }
-
-// field at X: Zeeman + demag (planar Hd) + exchange + anisotropy; also returns the unscaled
-// Laplacian
-__device__ __forceinline__ F3 field_at(const AdjArgs& a, const CellMat& cm, const float* X, const float* Hd, size_t n, size_t idx,
-	int i, int j, int k, float Ms, F3& lap)
-{
-	F3 H = (a.modules & BM_MOD_ZEEMAN) ? F3{ a.Hz[0], a.Hz[1], a.Hz[2] } : F3{ 0.f, 0.f, 0.f };
-	if (a.modules & BM_MOD_DEMAG) H = H + F3{ Hd[idx], Hd[n + idx], Hd[2 * n + idx] };
-	lap = F3{ 0.f, 0.f, 0.f };
-	if (a.modules & BM_MOD_EXCHANGE) { lap = lap_at(X, a, idx, i, j, k); H = H + cex(cm.A, Ms) * lap; }
-	if (a.modules & BM_MOD_ANIS_UNI) {
-		const F3 e{ a.ea[0], a.ea[1], a.ea[2] };
-		const float d = dot(ld3(X, idx), e) / Ms;
-		H = H + ((2.f / ((float)kMU0 * Ms)) * d * (cm.K1 + 2.f * a.K2 * (1.f - d * d))) * e;
-	}
-	return H;
-}
-
-__device__ __forceinline__ void cell_ijk(const AdjArgs& a, size_t idx, int& i, int& j, int& k)
-{
-	i = (int)(idx % a.nx); j = (int)((idx / a.nx) % a.ny); k = (int)(idx / ((size_t)a.nx * a.ny));
-}
 
 __global__ void k_init(float* M, const float* Ms, const float* m0, size_t n)
 {
@@ -125,8 +43,7 @@ __global__ void k_init(float* M, const float* Ms, const float* m0, size_t n)
 		st3(M, i, Ms[i] * ld3(m0, i));
 }
 
-// Forward stage S of the step from Mn: k = f(X); S < 3: acc (=, +=) w_S k, Xn = Mn + c_S dt k;
-// S == 3: Y = Mn + dt/6 (acc + k) (stored when Yout), Mnext = Ms Y / |Y|.
+// Forward stage S of the step from Mn (fwd_cell).
 template <int S>
 __global__ void __launch_bounds__(kAB) k_fwd(AdjArgs a, const float* __restrict__ X, const float* __restrict__ Hd, const float* __restrict__ Mn,
 	float* __restrict__ acc, float* __restrict__ Xn, float* __restrict__ Yout, float* __restrict__ Mnext, float dt)
@@ -134,23 +51,7 @@ __global__ void __launch_bounds__(kAB) k_fwd(AdjArgs a, const float* __restrict_
 	const size_t n = (size_t)a.nx * a.ny * a.nz;
 	for (size_t idx = blockIdx.x * (size_t)blockDim.x + threadIdx.x; idx < n; idx += (size_t)gridDim.x * blockDim.x) {
 		int i, j, k; cell_ijk(a, idx, i, j, k);
-		const float Ms = a.Ms[idx];
-		const CellMat cm = adj_mat(a, k);
-		F3 lap;
-		const F3 m = ld3(X, idx);
-		const F3 H = field_at(a, cm, X, Hd, n, idx, i, j, k, Ms, lap);
-		const F3 mxh = cross(m, H);
-		const float iMs = 1.f / Ms;
-		const F3 mu{ m.x * iMs, m.y * iMs, m.z * iMs };
-		const F3 f = pre_llg(a, cm.alpha) * (mxh + cm.alpha * cross(mu, mxh));
-		if (S == 0) { st3(acc, idx, f); st3(Xn, idx, ld3(Mn, idx) + (dt / 2) * f); }
-		else if (S == 1) { st3(acc, idx, ld3(acc, idx) + 2.f * f); st3(Xn, idx, ld3(Mn, idx) + (dt / 2) * f); }
-		else if (S == 2) { st3(acc, idx, ld3(acc, idx) + 2.f * f); st3(Xn, idx, ld3(Mn, idx) + dt * f); }
-		else {
-			const F3 Y = ld3(Mn, idx) + (dt / 6) * (ld3(acc, idx) + f);
-			if (Yout) st3(Yout, idx, Y);
-			st3(Mnext, idx, (Ms / norm(Y)) * Y);
-		}
+		fwd_put<S>(fwd_cell<S>(a, X, ld_planar(a.modules & BM_MOD_DEMAG ? Hd : nullptr, n, idx), Mn, acc, dt, idx, i, j, k), acc, Xn, Yout, Mnext, idx);
 	}
 }
 
@@ -182,13 +83,9 @@ __global__ void k_final(const float* M, const float* mt, const float* Ms, size_t
 __global__ void k_adj_renorm(const float* Y, const float* Ms, const float* lam, float* lamY, float* lacc, double* gMs, size_t n)
 {
 	for (size_t i = blockIdx.x * (size_t)blockDim.x + threadIdx.x; i < n; i += (size_t)gridDim.x * blockDim.x) {
-		const F3 y = ld3(Y, i);
-		const float nr = norm(y);
-		const F3 yh = (1.f / nr) * y;
-		const F3 l = ld3(lam, i);
-		const float yl = dot(yh, l);
-		gMs[i] += (double)yl;
-		const F3 ly = (Ms[i] / nr) * (l - yl * yh);
+		double g = 0;
+		const F3 ly = renorm_cell(Y, Ms[i], ld3(lam, i), g, i);
+		gMs[i] += g;
 		st3(lamY, i, ly);
 		st3(lacc, i, ly);
 	}
@@ -206,35 +103,12 @@ __global__ void __launch_bounds__(kAB) k_vjp_a(AdjArgs a, const float* __restric
 	double gz[4] = { 0, 0, 0, 0 };
 	for (size_t idx = blockIdx.x * (size_t)kAB + threadIdx.x; idx < n; idx += (size_t)gridDim.x * kAB) {
 		int i, j, k; cell_ijk(a, idx, i, j, k);
-		const float Ms = a.Ms[idx];
-		const CellMat cm = adj_mat(a, k);
-		const float pr = pre_llg(a, cm.alpha), al = cm.alpha;
-		F3 lap;
-		const F3 m = ld3(X, idx);
-		const F3 H = field_at(a, cm, X, Hd, n, idx, i, j, k, Ms, lap);
 		F3 w = ((dt / 6) * wS) * ld3(lamY, idx);
 		if (lxn) w = w + (cS * dt) * ld3(lxn, idx);
-		const float mh = dot(m, H), mw = dot(m, w), hw = dot(H, w), mm = dot(m, m);
-		F3 d = pr * (cross(H, w) + (al / Ms) * (mh * w + mw * H - (2.f * hw) * m));
-		const F3 uu = pr * (cross(w, m) + (al / Ms) * (mw * m - mm * w));
-		const float ce = cex(cm.A, Ms);
-		double g = -(double)pr * (double)al / ((double)Ms * Ms) * (double)dot(cross(m, cross(m, H)), w);
-		if (a.modules & BM_MOD_EXCHANGE) g += (double)dot(uu, lap) * (-2.0 * (double)ce / (double)Ms);
-		if (a.modules & BM_MOD_ANIS_UNI) {
-			// H_an = 2/mu0 s (K1 + 2K2 - 2K2 s^2/Ms^2)/Ms^2 e with s = m.e: its Jacobian is
-			// 2/(mu0 Ms^2) (K1 + 2K2 - 6K2 d^2) e e^T (d = s/Ms), its Ms derivative
-			// 2/mu0 s e (-2K1 - 4K2 + 8K2 d^2)/Ms^3
-			const F3 e{ a.ea[0], a.ea[1], a.ea[2] };
-			const float sm = dot(m, e), dd = sm / Ms, ue = dot(uu, e);
-			d = d + ((2.f / ((float)kMU0 * Ms * Ms)) * (cm.K1 + 2.f * a.K2 - 6.f * a.K2 * dd * dd) * ue) * e;
-			g += 2.0 / kMU0 * (double)sm * (double)ue * (-2.0 * cm.K1 - 4.0 * a.K2 + 8.0 * a.K2 * (double)dd * dd) / ((double)Ms * Ms * Ms);
-		}
-		st3(lx, idx, d);
-		st3(u, idx, uu);
-		st3(cu, idx, ce * uu);
+		double g = 0;
+		const VjpCell c = vjp_a_cell(a, X, ld_planar(a.modules & BM_MOD_DEMAG ? Hd : nullptr, n, idx), w, g, gz, idx, i, j, k);
+		st3(lx, idx, c.lx); st3(u, idx, c.u); st3(cu, idx, c.cu);
 		gMs[idx] += g;
-		gz[0] += (double)(dot(uu, F3{ a.dir[0], a.dir[1], a.dir[2] }) * a.sc);
-		gz[1] += (double)(uu.x * a.tz); gz[2] += (double)(uu.y * a.tz); gz[3] += (double)(uu.z * a.tz);
 	}
 	for (int c = 0; c < 4; c++) red[c][threadIdx.x] = gz[c];
 	__syncthreads();
@@ -252,9 +126,7 @@ __global__ void __launch_bounds__(kAB) k_vjp_b(AdjArgs a, const float* __restric
 	const size_t n = (size_t)a.nx * a.ny * a.nz;
 	for (size_t idx = blockIdx.x * (size_t)kAB + threadIdx.x; idx < n; idx += (size_t)gridDim.x * kAB) {
 		int i, j, k; cell_ijk(a, idx, i, j, k);
-		F3 v = ld3(lx, idx);
-		if (a.modules & BM_MOD_DEMAG) v = v + F3{ Nu[idx], Nu[n + idx], Nu[2 * n + idx] };
-		if (a.modules & BM_MOD_EXCHANGE) v = v + lap_at(cu, a, idx, i, j, k);
+		const F3 v = vjp_b_cell(a, ld_planar(a.modules & BM_MOD_DEMAG ? Nu : nullptr, n, idx), cu, ld3(lx, idx), idx, i, j, k);
 		st3(lx, idx, v);
 		st3(lacc, idx, ld3(lacc, idx) + v);
 	}
@@ -296,8 +168,11 @@ struct bm_adj_s {
 	float* Xs = nullptr;          // stage inputs without tape: 3 x 3n
 	float* lam = nullptr; float* lamY = nullptr; float* lacc = nullptr; float* lx = nullptr; float* lxn = nullptr;
 	float* u = nullptr; float* cu = nullptr; float* Nu = nullptr;
+	float* cu2 = nullptr;         // row kernels: c u of the stage before (its neighbours are still read)
 	double* gMs = nullptr;
-	double* part = nullptr;       // per-block partials: loss (grid), then 4 Zeeman sums per block
+	double* part = nullptr;       // per-block partials: loss (grid), then 4 Zeeman sums per block (npart)
+	int npart = 0;                // blocks of the plain kernels or work items of the row kernels, the larger
+	int ncu = 256;
 	double* h_part = nullptr;     // pinned
 	const float* m0 = nullptr; const float* mt = nullptr;
 	bool forward_done = false;
@@ -346,10 +221,75 @@ size_t n3(bm_adj_s* o) { return o->n * 3; }
 float* tX(bm_adj_s* o, int q, int s) { return o->tape + ((size_t)q * 5 + s) * n3(o); }                 // s = 0..3 stage inputs, 4 = Y
 float* tH(bm_adj_s* o, int q, int s) { return o->tape + (size_t)o->K * 5 * n3(o) + ((size_t)q * 4 + s) * n3(o); }
 
+// The evaluations go through the row kernels: demag on, open x with rows of N.x / 2 cells and few of them
+// (the rule of the split x passes).  Measured at 128x128x4, 8 steps forward and
+// backward: 2.49 -> 1.96 ms.
+bool use_rows(const bm_adj_s* o)
+{
+	if (!(o->p.modules & BM_MOD_DEMAG)) return false;
+	if (o->ml) { int mp[2]; mlayer_pbc(o->ml, mp); if (mp[0]) return false; }
+	else if (o->demag->full[0] || o->demag->Nx != 2 * o->nx) return false;
+	return xs_few_rows(o->nx, o->ny, o->nz, o->ncu);
+}
+
+AdjRow row_of(bm_adj_s* o)
+{
+	if (o->ml) { const MlView v = mlayer_view(o->ml); return AdjRow{ v.Sx, v.ntl, (float)(1.0 / ((double)v.Nx * v.Ny)) }; }
+	const bm_demag_s* d = o->demag;
+	return AdjRow{ d->Sx, d->ntl, (float)(1.0 / ((double)d->Nx * d->Ny * d->Nz)) };
+}
+
+int x_forward(bm_adj_s* o, const float* M, hipStream_t st) { return o->ml ? mlayer_fwd_x(o->ml, M, st) : demag_fwd_x(o->demag, M, st); }
+
+// one forward step with the row kernels: the spectra hold the x transform of Mn, and of Mnext afterwards
+int fwd_step_rows(bm_adj_s* o, int step, const float* Mn, float* Mnext, int q, hipStream_t st)
+{
+	const AdjArgs a = adj_args(o, step);
+	const AdjRow r = row_of(o);
+	const float* X = Mn;
+	if (q >= 0) BM_HIP(hipMemcpyAsync(tX(o, q, 0), Mn, n3(o) * sizeof(float), hipMemcpyDeviceToDevice, st));
+	for (int s = 0; s < 4; s++) {
+		int rc = o->ml ? mlayer_mid(o->ml, st) : demag_mid(o->demag, st);
+		if (rc) return rc;
+		AdjFwd f{ X, Mn, o->acc, nullptr, nullptr, Mnext, q >= 0 ? tH(o, q, s) : nullptr, (float)o->dt };
+		if (s < 3) f.Xn = q >= 0 ? tX(o, q, s + 1) : o->Xs + (size_t)s * n3(o);
+		else if (q >= 0) f.Yout = tX(o, q, 4);
+		if ((rc = adj_row_fwd(s, a, r, f, st))) return rc;
+		X = f.Xn;
+	}
+	return BM_OK;
+}
+
+// adjoint of one step with the row kernels; begin: the first of a segment (lam holds dL/dM of its end),
+// end: the last (lam receives dL/dM of its start), otherwise the steps run into each other
+int adj_step_rows(bm_adj_s* o, int step, int q, bool begin, bool end, hipStream_t st)
+{
+	static const float wgt[4] = { 1, 2, 2, 1 }, cst[3] = { 0.5f, 0.5f, 1.0f };
+	const AdjRow r = row_of(o);
+	AdjBwd w{};
+	w.lam = o->lam; w.lamY = o->lamY; w.lacc = o->lacc; w.lx = o->lx; w.gMs = o->gMs; w.apart = o->part + o->grid; w.dt = (float)o->dt;
+	auto at = [&](int qq, int s) {
+		w.Y = tX(o, qq, 4); w.X = tX(o, qq, s); w.Hd = tH(o, qq, s);
+		w.wS = wgt[s]; w.cS = s < 3 ? cst[s] : 0.f;
+		w.cu_in = o->cu; w.cu_out = o->cu2;
+		std::swap(o->cu, o->cu2);
+	};
+	int rc = BM_OK;
+	if (begin) { at(q, 3); rc = adj_row_bwd(false, true, true, adj_args(o, step), r, w, st); }
+	for (int s = 3; s >= 0 && !rc; s--) {
+		if ((rc = o->ml ? mlayer_mid(o->ml, st, 1) : demag_mid(o->demag, st))) return rc;
+		if (s > 0) { at(q, s - 1); rc = adj_row_bwd(true, false, true, adj_args(o, step), r, w, st); }
+		else if (end) { at(q, 0); rc = adj_row_bwd(true, false, false, adj_args(o, step), r, w, st); }
+		else { at(q - 1, 3); rc = adj_row_bwd(true, true, true, adj_args(o, step - 1), r, w, st); }
+	}
+	return rc;
+}
+
 // one forward step from Mn into Mnext; with taping (q >= 0) the stage inputs, their demag
 // fields and Y go to tape slot q
 int fwd_step(bm_adj_s* o, int step, const float* Mn, float* Mnext, int q, hipStream_t st)
 {
+	if (use_rows(o)) return fwd_step_rows(o, step, Mn, Mnext, q, st);
 	const AdjArgs a = adj_args(o, step);
 	const float dt = (float)o->dt;
 	const float* X = Mn;
@@ -375,8 +315,9 @@ int fwd_step(bm_adj_s* o, int step, const float* Mn, float* Mnext, int q, hipStr
 }
 
 // adjoint of one step with tape slot q: lam (dL/dM_{step+1}) -> lam (dL/dM_step)
-int adj_step(bm_adj_s* o, int step, int q, hipStream_t st)
+int adj_step(bm_adj_s* o, int step, int q, bool begin, bool end, hipStream_t st)
 {
+	if (use_rows(o)) return adj_step_rows(o, step, q, begin, end, st);
 	const AdjArgs a = adj_args(o, step);
 	const float dt = (float)o->dt;
 	const dim3 g(o->grid), b(kAB);
@@ -401,7 +342,7 @@ void free_all(bm_adj_s* o)
 {
 	if (o->done) (void)hipEventDestroy(o->done);
 	if (o->own) (void)hipStreamDestroy(o->own);
-	float* fl[] = { o->ck, o->tape, o->Mw, o->acc, o->Hd, o->Xs, o->lam, o->lamY, o->lacc, o->lx, o->lxn, o->u, o->cu, o->Nu };
+	float* fl[] = { o->ck, o->tape, o->Mw, o->acc, o->Hd, o->Xs, o->lam, o->lamY, o->lacc, o->lx, o->lxn, o->u, o->cu, o->cu2, o->Nu };
 	for (float* p : fl) if (p) (void)hipFree(p);
 	if (o->gMs) (void)hipFree(o->gMs);
 	if (o->part) (void)hipFree(o->part);
@@ -424,6 +365,8 @@ extern "C" int bm_adj_create(int nx, int ny, int nz, double hx, double hy, doubl
 	o->dt = dt; o->nsteps = nsteps; o->K = std::min(ckpt_every, nsteps);
 	o->nck = (nsteps + o->K - 1) / o->K + 1;
 	o->grid = (int)std::max<size_t>(1, std::min<size_t>((o->n + kAB - 1) / kAB, (size_t)device_cu_count() * 8));
+	o->ncu = device_cu_count();
+	o->npart = std::max(o->grid, xs_few_rows(nx, ny, nz, o->ncu) ? xs_parts(nx, ny, nz) : 0);
 	const size_t b3 = n3(o) * sizeof(float);
 	bool ok = hipMalloc(&o->ck, (size_t)o->nck * b3) == hipSuccess
 		&& hipMalloc(&o->tape, (size_t)o->K * 9 * b3) == hipSuccess
@@ -431,10 +374,10 @@ extern "C" int bm_adj_create(int nx, int ny, int nz, double hx, double hy, doubl
 		&& hipMalloc(&o->Hd, b3) == hipSuccess && hipMalloc(&o->Xs, 3 * b3) == hipSuccess
 		&& hipMalloc(&o->lam, b3) == hipSuccess && hipMalloc(&o->lamY, b3) == hipSuccess && hipMalloc(&o->lacc, b3) == hipSuccess
 		&& hipMalloc(&o->lx, b3) == hipSuccess && hipMalloc(&o->lxn, b3) == hipSuccess
-		&& hipMalloc(&o->u, b3) == hipSuccess && hipMalloc(&o->cu, b3) == hipSuccess && hipMalloc(&o->Nu, b3) == hipSuccess
+		&& hipMalloc(&o->u, b3) == hipSuccess && hipMalloc(&o->cu, b3) == hipSuccess && hipMalloc(&o->cu2, b3) == hipSuccess && hipMalloc(&o->Nu, b3) == hipSuccess
 		&& hipMalloc(&o->gMs, o->n * sizeof(double)) == hipSuccess
-		&& hipMalloc(&o->part, 5 * (size_t)o->grid * sizeof(double)) == hipSuccess
-		&& hipHostMalloc(&o->h_part, 5 * (size_t)o->grid * sizeof(double)) == hipSuccess;
+		&& hipMalloc(&o->part, ((size_t)o->grid + 4 * (size_t)o->npart) * sizeof(double)) == hipSuccess
+		&& hipHostMalloc(&o->h_part, ((size_t)o->grid + 4 * (size_t)o->npart) * sizeof(double)) == hipSuccess;
 	if (!ok) { free_all(o); delete o; return fail(BM_ERR_NOMEM, "bm_adj_create: device memory"); }
 	*out = o;
 	return BM_OK;
@@ -457,7 +400,7 @@ int fwd_begin(bm_adj_s* o, const float* m0, const float* mt, hipStream_t st)
 	o->m0 = m0; o->mt = mt;
 	hipLaunchKernelGGL(k_init, dim3(o->grid), dim3(kAB), 0, st, o->ck, o->Ms, m0, o->n);
 	o->cur = o->ck;
-	return BM_OK;
+	return use_rows(o) ? x_forward(o, o->cur, st) : BM_OK;
 }
 
 // step s, checkpointing every K steps and at the end
@@ -491,7 +434,7 @@ int bwd_begin(bm_adj_s* o, hipStream_t st)
 {
 	float* Mfin = o->ck + (size_t)(o->nck - 1) * n3(o);
 	hipLaunchKernelGGL(k_final, dim3(o->grid), dim3(kAB), 0, st, Mfin, o->mt, o->Ms, o->n, o->lam, o->gMs);
-	BM_HIP(hipMemsetAsync(o->part + o->grid, 0, 4 * (size_t)o->grid * sizeof(double), st));
+	BM_HIP(hipMemsetAsync(o->part + o->grid, 0, 4 * (size_t)o->npart * sizeof(double), st));
 	return BM_OK;
 }
 
@@ -499,7 +442,10 @@ int bwd_begin(bm_adj_s* o, hipStream_t st)
 int bwd_recompute(bm_adj_s* o, int sg, int s, hipStream_t st)
 {
 	const int s0 = sg * o->K;
-	if (s == s0) o->cur = o->ck + (size_t)sg * n3(o);
+	if (s == s0) {
+		o->cur = o->ck + (size_t)sg * n3(o);
+		if (use_rows(o)) if (int rc = x_forward(o, o->cur, st)) return rc;
+	}
 	float* next = (o->cur == o->Mw) ? o->Mw + n3(o) : o->Mw;
 	int rc = fwd_step(o, s, o->cur, next, s - s0, st);
 	o->cur = next;
@@ -511,14 +457,14 @@ int bwd_end(bm_adj_s* o, float* gMs_out, hipStream_t st)
 	const dim3 g(o->grid), b(kAB);
 	hipLaunchKernelGGL(k_m0_term, g, b, 0, st, o->m0, o->lam, o->gMs, o->n);
 	hipLaunchKernelGGL(k_to_float, g, b, 0, st, o->gMs, gMs_out, o->n);
-	BM_HIP(hipMemcpyAsync(o->h_part, o->part + o->grid, 4 * (size_t)o->grid * sizeof(double), hipMemcpyDeviceToHost, st));
+	BM_HIP(hipMemcpyAsync(o->h_part, o->part + o->grid, 4 * (size_t)o->npart * sizeof(double), hipMemcpyDeviceToHost, st));
 	return BM_OK;
 }
 
 void bwd_finish(bm_adj_s* o, double* gamp)
 {
 	for (int c = 0; c < 4; c++) o->gz[c] = 0;
-	for (int q = 0; q < o->grid; q++) for (int c = 0; c < 4; c++) o->gz[c] += o->h_part[4 * q + c];
+	for (int q = 0; q < o->npart; q++) for (int c = 0; c < 4; c++) o->gz[c] += o->h_part[4 * q + c];
 	if (gamp) *gamp = o->gz[0];
 }
 
@@ -591,7 +537,7 @@ extern "C" int bm_adj_backward(bm_adj_t o, float* gMs_out, double* gamp, void* s
 	for (int sg = o->nck - 2; sg >= 0 && !rc; sg--) {
 		const int s0 = sg * o->K, s1 = std::min(o->nsteps, s0 + o->K);
 		for (int s = s0; s < s1 && !rc; s++) rc = bwd_recompute(o, sg, s, st);
-		for (int s = s1 - 1; s >= s0 && !rc; s--) rc = adj_step(o, s, s - s0, st);
+		for (int s = s1 - 1; s >= s0 && !rc; s--) rc = adj_step(o, s, s - s0, s == s1 - 1, s == s0, st);
 	}
 	if (!rc) rc = bwd_end(o, gMs_out, st);
 	if (rc) return rc;
@@ -639,7 +585,7 @@ extern "C" int bm_adj_batch_backward(int count, const bm_adj_t* hs, float* const
 		for (int s = s0; s < s1 && !rc; s++)
 			for (int b = 0; b < count && !rc; b++) rc = bwd_recompute(hs[b], sg, s, hs[b]->own);
 		for (int s = s1 - 1; s >= s0 && !rc; s--)
-			for (int b = 0; b < count && !rc; b++) rc = adj_step(hs[b], s, s - s0, hs[b]->own);
+			for (int b = 0; b < count && !rc; b++) rc = adj_step(hs[b], s, s - s0, s == s1 - 1, s == s0, hs[b]->own);
 	}
 	for (int b = 0; b < count && !rc; b++) rc = bwd_end(hs[b], gMs_out[b], hs[b]->own);
 	if (!rc) rc = batch_join(hs, count, st);

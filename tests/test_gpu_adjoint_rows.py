@@ -1,0 +1,29 @@
+"""The adjoint's row kernels (one kernel between two convolutions' middle passes) at the edges of
+their row groups: the shortest rows, rows of part of a wave and of a whole one, the fourth wave of
+the per-cell work, radix-3 rows, and row counts that leave the last group ragged."""
+import numpy as np
+import pytest
+import torch
+
+from boris2_amd import api
+from test_gpu_adjoint import oracle_grads, problem
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("n", [(8, 6, 2), (32, 24, 1), (96, 6, 2), (128, 12, 1), (128, 6, 2), (256, 6, 2), (512, 6, 1)])
+def test_adjoint_rows_match_oracle(gpu, n):
+    n, p, Ms, m0, mt = problem(n, seed=sum(n))
+    dt, steps = 250e-15, 8
+    L0, g0, ga0 = oracle_grads(n, p, Ms, m0, mt, dt, steps)
+    r = api.RK4Adjoint(n, (4e-9,) * 3, p, torch.tensor(Ms, dtype=torch.float32), dt, steps, 3)
+    L, _ = r.forward(torch.tensor(m0, dtype=torch.float32), torch.tensor(mt, dtype=torch.float32))
+    g, ga = r.backward()
+    g = g.cpu().numpy().astype(np.float64)
+    eg, ea = np.linalg.norm(g - g0) / np.linalg.norm(g0), abs(ga - ga0) / abs(ga0)
+    print(f"{n}: loss {abs(L - L0):.2e}, dL/dMs rel L2 {eg:.2e}, dL/damp rel {ea:.2e}")
+    # the bounds of the 40-step comparison of the same problem (FP32 forward's departure, linear in the steps)
+    assert abs(L - L0) <= 1e-6
+    assert eg <= 5e-5
+    assert ea <= 5e-5
+    r.close()
