@@ -498,7 +498,8 @@ bool row_path(const bm_ode_s* o)
 // 512x512x3 435 -> 392, 384x384x6 586 -> 506.
 bool row_stack(const bm_ode_s* o)
 {
-	if (!o->ml || !o->row_env || o->speedup || o->pbc[0] || o->pbc[1] || o->pbc[2]) return false;
+	// a field function may use the stack's handle, whose spectra the row kernel would rely on
+	if (!o->ml || !o->row_env || o->speedup || o->ext_fn || o->pbc[0] || o->pbc[1] || o->pbc[2]) return false;
 	int mp[2];
 	mlayer_pbc(o->ml, mp);
 	return !mp[0] && !mp[1] && xs_few_rows(o->nx, o->ny, o->nz, o->ncu, true);

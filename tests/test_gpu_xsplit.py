@@ -99,3 +99,26 @@ def test_layer_stack_rows_match_the_separate_passes(gpu, monkeypatch, nx, ny, gr
         out.append(s.M.cpu().numpy().astype(np.float64))
         s.close()
     assert rel(out[0], out[1]) <= 5e-7
+
+
+def test_stack_field_function_may_use_the_stacks_handle(gpu):
+    """A field function that convolves with the stack's own multilayer handle (for an energy, say)
+    must not disturb the run: the same bits as with one that leaves the handle alone."""
+    L, nx, ny = 3, 64, 8
+    p = api.FMParams(Ms=8e5, A=1.3e-11, alpha=0.1, modules=api.BM_MOD_DEMAG | api.BM_MOD_EXCHANGE)
+    M0 = api.random_magnetisation(L * nx * ny, 8e5, 4).astype(np.float32)
+    other = torch.from_numpy(M0[::-1].copy()).cuda()
+    out = []
+    for use in (False, True):
+        s = api.LayerStackSolver(api.BM_EVAL_RK4, nx, ny, 4e-9, 4e-9, [4e-9] * L, [4e-9 * l for l in range(L)], p, M0=M0)
+
+        def field(M):
+            if use:
+                s.mlayer.convolute(other)
+            return torch.full_like(M, 1e4)
+        s.set_extra_field(field)
+        s.set_dt(2e-14)
+        s.run_to_iteration(3)
+        out.append(s.M.clone())
+        s.close()
+    assert torch.equal(out[0], out[1])
