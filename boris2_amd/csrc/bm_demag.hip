@@ -17,6 +17,8 @@
 //        P4 y-IFFT     S: Ny in -> Sx: ny out
 //        P5 x-C2R      Sx -> H (planar or AoS, set or add), scaled by 1/(Nx Ny Nz)
 //   2D:  P1, P2' (y-FFT * K * y-IFFT per kx line of Sx, 3 components, in place), P5.
+// Where the column pass serves the mesh (bm_col.hip) it replaces P2 + P3 + P4 and P2'; x passes
+// with few rows take the form of bm_xsplit.h.
 //
 // Kernel setup runs once on the GPU in FP64 (Newell f/g grids, 27-point stencil or
 // far-field series, mirror placement, three real-input FFT passes) and stores FP32
@@ -999,10 +1001,11 @@ template <int NY, int NZ> int batch_yzy_t(LaunchShape sh, const PassBatch* h_tab
 
 // the fused thin-mesh pass serves this mesh (open y and z, N.z 4 or 8, a power-of-two N.y
 // with a schedule that fits).  By default only for N.z = 4 (two planes, held in registers with
-// the radix-4 schedules) from 128 x 128 cells per plane: measured (RK4 steps, against the
-// separate passes) 128x128x2 0.221 -> 0.207 ms, 256x256x2 0.256 -> 0.215, 512x512x2 0.364 ->
-// 0.284, 1024x1024x2 0.994 -> 0.885 (N.y 2048: the LDS line buffer); for N.z = 8 (the LDS line
-// buffer) 256x256x4 and 1024x512x4 within +-2 % either way, so not by default.
+// the radix-4 schedules) from 128 x 128 cells per plane, and there only where the column pass
+// is not the better one (use_col).  Against the separate passes (RK4 steps) 128x128x2 0.221 ->
+// 0.207 ms, 256x256x2 0.256 -> 0.215, 512x512x2 0.364 -> 0.284, 1024x1024x2 0.994 -> 0.885
+// (N.y 2048: the LDS line buffer); for N.z = 8 (the LDS line buffer) 256x256x4 and 1024x512x4
+// within +-2 % either way, so not by default.
 bool yzy_ok(const bm_demag_s* d)
 {
 	if (!d->yzy || d->is2d || d->full[1] || d->full[2] || (d->Nz != 4 && d->Nz != 8)) return false;
