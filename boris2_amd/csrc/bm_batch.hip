@@ -88,7 +88,7 @@ struct bm_batch_s {
 	// RKDP54: per-mesh step control (device) and its host copy (pinned, refreshed by runs)
 	BatchCtl* d_ctl = nullptr;
 	BatchCtl* h_ctl = nullptr;
-	unsigned* d_lte = nullptr;
+	unsigned long long* d_lte = nullptr;
 	float* Hd = nullptr;           // planar per mesh: 3 * ncell[b] at 3 * off[b]
 	// pass groups and their tables
 	std::vector<Group> gx, gy, gz, gy2, gml;
@@ -220,7 +220,7 @@ __global__ void k_batch_fields(const StageArgs* __restrict__ tab, int nb)
 // RKDP54 step control after stage 0, one thread per mesh: the plain integrator's stage-0
 // branch (primed check, SetAdaptiveTimeStep, restore on rejection) on the device.  The new
 // dT goes into both stage tables (read in place by the stage kernels of this replay).
-__global__ void k_rkdp_control(BatchCtl* ctl, unsigned* lte, StageArgs* t0, StageArgs* t1, int nb)
+__global__ void k_rkdp_control(BatchCtl* ctl, unsigned long long* lte, StageArgs* t0, StageArgs* t1, int nb)
 {
 	const int b = blockIdx.x * blockDim.x + threadIdx.x;
 	if (b >= nb) return;
@@ -228,7 +228,7 @@ __global__ void k_rkdp_control(BatchCtl* ctl, unsigned* lte, StageArgs* t0, Stag
 	if (!c.active) { c.skip = 1; return; }
 	c.skip = 0;
 	if (c.primed) {
-		c.lte = (double)__uint_as_float(lte[b]);
+		c.lte = (double)__uint_as_float((unsigned)lte[b]);
 		if (c.dT_min != c.dT_max) {
 			if (c.lte > c.err_high_fail && c.dT > c.dT_min) {
 				c.time -= c.dT; c.iteration--;
@@ -251,7 +251,7 @@ __global__ void k_rkdp_control(BatchCtl* ctl, unsigned* lte, StageArgs* t0, Stag
 		}
 	}
 	else c.primed = 1;
-	lte[b] = 0u;
+	lte[b] = 0;
 	t0[b].dT = (float)c.dT;
 	t1[b].dT = (float)c.dT;
 }
@@ -807,8 +807,8 @@ extern "C" int bm_batch_create_layers(int method, int nmesh, const int* n3, cons
 			// the reference's RKDP54 defaults (Boris/DiffEq_CommonBase_Control.cpp:10-140)
 			ok = hipHostMalloc(&o->h_ctl, nmesh * sizeof(BatchCtl)) == hipSuccess
 				&& hipMalloc(&o->d_ctl, nmesh * sizeof(BatchCtl)) == hipSuccess
-				&& hipMalloc(&o->d_lte, nmesh * sizeof(unsigned)) == hipSuccess
-				&& hipMemset(o->d_lte, 0, nmesh * sizeof(unsigned)) == hipSuccess;
+				&& hipMalloc(&o->d_lte, nmesh * sizeof(*o->d_lte)) == hipSuccess
+				&& hipMemset(o->d_lte, 0, nmesh * sizeof(*o->d_lte)) == hipSuccess;
 			if (ok) {
 				for (int b = 0; b < nmesh; b++) {
 					BatchCtl& c = o->h_ctl[b];

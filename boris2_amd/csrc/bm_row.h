@@ -102,7 +102,7 @@ __global__ void __launch_bounds__(BS) k_row(StageArgs a, float2* Sx, int ntl, in
 			}
 		}
 	}
-	if (stage_has_lte<METHOD, STEP>()) block_max_to<BS>(lte_loc, a.lte);
+	if (stage_has_lte<METHOD, STEP>()) block_max_to<BS>(lte_loc, a);
 }
 
 // Wave-independent variant for rows whose x transform is exactly one wavefront (HX = 512:
@@ -216,7 +216,7 @@ __global__ void __launch_bounds__(kXBlock) k_roww(StageArgs a, float2* Sx, int n
 			}
 		}
 	}
-	if (stage_has_lte<METHOD, STEP>()) block_max_to<kXBlock>(lte_loc, a.lte);
+	if (stage_has_lte<METHOD, STEP>()) block_max_to<kXBlock>(lte_loc, a);
 }
 
 // What the row kernel works on: the x-side spectra of nz planes of ny rows (a mesh's, or a stack's

@@ -101,7 +101,8 @@ struct StageArgs {
 	const float* Ms_map;
 	float* Heff_out;        // optional AoS copy of the effective field
 	const float* Hext;      // optional AoS field of other modules, added to the effective field
-	unsigned* lte;          // max lte as float bits
+	unsigned long long* lte; // max lte as float bits, below the step's tag lte_tag
+	unsigned lte_tag;       // 0 where the word is cleared for every estimate (batches)
 	int nx, ny, nz;
 	int per;                // periodic exchange along x, y, z: bits 0, 1, 2
 	float ihx2, ihy2, ihz2; // 1 / h^2 per axis
@@ -178,7 +179,7 @@ enum { M_RKDP = 0, M_RK4 = 1, M_TEULER = 2, M_AHEUN = 3 };
 // queueing on one word held the stage up (RKDP54 stage 0 of 256x256x16 cells, 4096 blocks: 58 us
 // against 24 to 29 us of the other stages).
 template <int NT = kBS>
-__device__ __forceinline__ void block_max_to(float v, unsigned* dst)
+__device__ __forceinline__ void block_max_to(float v, const StageArgs& a)
 {
 	__shared__ float red[NT / 64];
 	for (int o = 32; o > 0; o >>= 1) v = fmaxf(v, __shfl_xor(v, o));
@@ -187,8 +188,8 @@ __device__ __forceinline__ void block_max_to(float v, unsigned* dst)
 	if (threadIdx.x == 0) {
 		float m = red[0];
 		for (int q = 1; q < NT / 64; q++) m = fmaxf(m, red[q]);
-		const unsigned u = __float_as_uint(m);
-		if (u > __hip_atomic_load(dst, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) atomicMax(dst, u);
+		const unsigned long long u = (unsigned long long)a.lte_tag << 32 | __float_as_uint(m);
+		if (u > __hip_atomic_load(a.lte, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) atomicMax(a.lte, u);
 	}
 }
 

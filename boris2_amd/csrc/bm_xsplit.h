@@ -264,7 +264,7 @@ __global__ void __launch_bounds__((XSplit<HX, xs_groups<HX, LAY>()>::BS)) k_rows
 			__syncthreads();
 		}
 	}
-	if (stage_has_lte<METHOD, STEP>()) block_max_to<X::BS>(lte_loc, a.lte);
+	if (stage_has_lte<METHOD, STEP>()) block_max_to<X::BS>(lte_loc, a);
 }
 
 } // namespace bm
