@@ -16,8 +16,9 @@ namespace bm {
 
 constexpr int kTw2Max = 8192, kTw3Max = 3072;
 
-struct Tw2Table { float v[2 * kTw2Max][2]; };
-struct Tw3Table { float v[2 * kTw3Max - 3][2]; };
+// 16-byte aligned: entries are read 8 bytes at a time
+struct alignas(16) Tw2Table { float v[2 * kTw2Max][2]; };
+struct alignas(16) Tw3Table { float v[2 * kTw3Max - 3][2]; };
 
 // cos and -sin of 2 pi j / D: the quarter turn nearest to j / D exactly, the rest (at most
 // pi / 4) by the Taylor series (the terms left out are below 1e-18)
@@ -60,6 +61,7 @@ static __device__ constexpr Tw3Table kTw3 = make_tw3();
 // the roots of denominator D (2^a or 3 2^a): entry j is exp(-2 pi i j / D), 0 <= j < D
 template <int D> __device__ __forceinline__ const float2* tw_roots()
 {
+	static_assert(alignof(Tw2Table) >= alignof(float2) && alignof(Tw3Table) >= alignof(float2), "entries are read as float2");
 	static_assert(D >= 1 && ((D & (D - 1)) == 0 ? D <= kTw2Max : D % 3 == 0 && ((D / 3) & (D / 3 - 1)) == 0 && D <= kTw3Max), "no roots of this order");
 	if constexpr ((D & (D - 1)) == 0) return reinterpret_cast<const float2*>(kTw2.v[D]);
 	else return reinterpret_cast<const float2*>(kTw3.v[D - 3]);
