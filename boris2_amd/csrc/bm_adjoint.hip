@@ -167,8 +167,7 @@ struct bm_adj_s {
 	float* Hd = nullptr;          // planar 3n (forward without tape)
 	float* Xs = nullptr;          // stage inputs without tape: 3 x 3n
 	float* lam = nullptr; float* lamY = nullptr; float* lacc = nullptr; float* lx = nullptr; float* lxn = nullptr;
-	float* u = nullptr; float* cu = nullptr; float* Nu = nullptr;
-	float* cu2 = nullptr;         // row kernels: c u of the stage before (its neighbours are still read)
+	float* u = nullptr; float* cu = nullptr; float* Nu = nullptr;   // row kernels: u is the second c u
 	double* gMs = nullptr;
 	double* part = nullptr;       // per-block partials: loss (grid), then 4 Zeeman sums per block (npart)
 	int npart = 0;                // blocks of the plain kernels or work items of the row kernels, the larger
@@ -271,8 +270,9 @@ int adj_step_rows(bm_adj_s* o, int step, int q, bool begin, bool end, hipStream_
 	auto at = [&](int qq, int s) {
 		w.Y = tX(o, qq, 4); w.X = tX(o, qq, s); w.Hd = tH(o, qq, s);
 		w.wS = wgt[s]; w.cS = s < 3 ? cst[s] : 0.f;
-		w.cu_in = o->cu; w.cu_out = o->cu2;
-		std::swap(o->cu, o->cu2);
+		// the stage before's c u is still read for its neighbours; u itself lives in the spectra here
+		w.cu_in = o->cu; w.cu_out = o->u;
+		std::swap(o->cu, o->u);
 	};
 	int rc = BM_OK;
 	if (begin) { at(q, 3); rc = adj_row_bwd(false, true, true, adj_args(o, step), r, w, st); }
@@ -342,7 +342,7 @@ void free_all(bm_adj_s* o)
 {
 	if (o->done) (void)hipEventDestroy(o->done);
 	if (o->own) (void)hipStreamDestroy(o->own);
-	float* fl[] = { o->ck, o->tape, o->Mw, o->acc, o->Hd, o->Xs, o->lam, o->lamY, o->lacc, o->lx, o->lxn, o->u, o->cu, o->cu2, o->Nu };
+	float* fl[] = { o->ck, o->tape, o->Mw, o->acc, o->Hd, o->Xs, o->lam, o->lamY, o->lacc, o->lx, o->lxn, o->u, o->cu, o->Nu };
 	for (float* p : fl) if (p) (void)hipFree(p);
 	if (o->gMs) (void)hipFree(o->gMs);
 	if (o->part) (void)hipFree(o->part);
@@ -374,7 +374,7 @@ extern "C" int bm_adj_create(int nx, int ny, int nz, double hx, double hy, doubl
 		&& hipMalloc(&o->Hd, b3) == hipSuccess && hipMalloc(&o->Xs, 3 * b3) == hipSuccess
 		&& hipMalloc(&o->lam, b3) == hipSuccess && hipMalloc(&o->lamY, b3) == hipSuccess && hipMalloc(&o->lacc, b3) == hipSuccess
 		&& hipMalloc(&o->lx, b3) == hipSuccess && hipMalloc(&o->lxn, b3) == hipSuccess
-		&& hipMalloc(&o->u, b3) == hipSuccess && hipMalloc(&o->cu, b3) == hipSuccess && hipMalloc(&o->cu2, b3) == hipSuccess && hipMalloc(&o->Nu, b3) == hipSuccess
+		&& hipMalloc(&o->u, b3) == hipSuccess && hipMalloc(&o->cu, b3) == hipSuccess && hipMalloc(&o->Nu, b3) == hipSuccess
 		&& hipMalloc(&o->gMs, o->n * sizeof(double)) == hipSuccess
 		&& hipMalloc(&o->part, ((size_t)o->grid + 4 * (size_t)o->npart) * sizeof(double)) == hipSuccess
 		&& hipHostMalloc(&o->h_part, ((size_t)o->grid + 4 * (size_t)o->npart) * sizeof(double)) == hipSuccess;

@@ -27,3 +27,22 @@ def test_adjoint_rows_match_oracle(gpu, n):
     assert eg <= 5e-5
     assert ea <= 5e-5
     r.close()
+
+
+def test_adjoint_holds_no_array_beyond_its_own(gpu):
+    """Device memory of an instance of 1 M cells: checkpoints (3), the tape of one step (9), the two
+    working states, acc, the field, three stage inputs and the eight arrays of the backward pass, 12
+    bytes a cell each, and 8 bytes a cell of dL/dMs, within a third of one array."""
+    n, cells = (1024, 1024, 1), 1 << 20
+    Ms = torch.full((cells,), 8e5, device="cuda")
+    p = api.FMParams(Ms=8e5, A=1.3e-11, alpha=0.1, modules=api.BM_MOD_EXCHANGE)
+    one = api.RK4Adjoint((8, 8, 1), (4e-9,) * 3, p, Ms[:64], 1e-14, 2, 1)     # the library's code is on the device
+    m = torch.ones(64, 3, device="cuda")
+    one.forward(m, m)
+    torch.cuda.synchronize()
+    free = torch.cuda.mem_get_info()[0]
+    r = api.RK4Adjoint(n, (4e-9,) * 3, p, Ms, 1e-14, 2, 1)
+    used = free - torch.cuda.mem_get_info()[0]
+    r.close(); one.close()
+    print(f"{used / cells:.2f} bytes a cell")
+    assert used <= (12 * (3 + 9 + 2 + 1 + 1 + 3 + 8) + 8 + 4) * cells
