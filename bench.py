@@ -79,6 +79,7 @@ def algorithmic_bytes(kind: str, n, N) -> float:
         "row_c2r_stage_r2c": (11 * half + 38 * 12.0 * cells) / 6,
         # x-R2C fused with the RKDP54 advance: M, E0 in; sM1, M1 out; spectra rows out
         "fwd_x_advance": 4 * 12.0 * cells + half,
+        "column_pass": 2 * half + (16.0 * NC * NYH if nz == 1 else kern),
     }[kind]
 
 

@@ -1210,10 +1210,9 @@ int bm::demag_mid(bm_demag_s* d, hipStream_t st)
 	const int nlines = 3 * d->nz * d->NC;
 	int rc;
 	if (use_col(d)) {
-		// the middle passes as one, timed as the 2D y or the z pass
-		prof_mark_begin(d->is2d ? PK_Y2D : PK_Z, st);
+		prof_mark_begin(PK_COL, st);
 		rc = launch_col(d->Ny, d->Nz, d->full[1], d->Sx, d->K, nullptr, d->nz, d->NC, d->NYH, d->ntl, d->full[1] ? d->Ny : d->ny, 0, d->ncu, st);
-		prof_mark_end(d->is2d ? PK_Y2D : PK_Z, st);
+		prof_mark_end(PK_COL, st);
 		return rc;
 	}
 	if (d->is2d) {

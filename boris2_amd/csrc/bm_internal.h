@@ -31,7 +31,7 @@ __device__ __forceinline__ void st_nt(float2* p, float x, float y)
 
 // Launch timing: when enabled (bm_prof_begin), every kernel launch of the hot path is
 // bracketed by HIP events on its own stream and tagged with its kind.
-enum ProfKind { PK_FWD_X = 0, PK_Y_FWD, PK_Z, PK_Y_INV, PK_INV_X, PK_Y2D, PK_STAGE, PK_ADVANCE, PK_ROW, PK_FWD_ADV, PK_ML_MULT, PK_COUNT };
+enum ProfKind { PK_FWD_X = 0, PK_Y_FWD, PK_Z, PK_Y_INV, PK_INV_X, PK_Y2D, PK_STAGE, PK_ADVANCE, PK_ROW, PK_FWD_ADV, PK_ML_MULT, PK_COL, PK_COUNT };
 void prof_mark_begin(int kind, hipStream_t st);
 void prof_mark_end(int kind, hipStream_t st);
 // self-demag coefficient (-N diagonal) of one cell of size hx x hy x hz (bm_tensor.cpp)

@@ -1152,10 +1152,9 @@ int bm::mlayer_mid(bm_mlayer_s* m, hipStream_t st, int tr)
 	const bool fy = m->pbc[1] > 0;
 	int rc;
 	if (!m->Kc && bm::col_ok(m->Ny, 0, L, m->NC, m->ncu)) {
-		// the y passes and the product as one, timed as the product
-		bm::prof_mark_begin(bm::PK_ML_MULT, st);
+		bm::prof_mark_begin(bm::PK_COL, st);
 		rc = bm::launch_col(m->Ny, 0, fy, m->Sx, m->K, m->kcol, L, m->NC, m->NYH, m->ntl, fy ? m->Ny : m->ny, tr, m->ncu, st);
-		bm::prof_mark_end(bm::PK_ML_MULT, st);
+		bm::prof_mark_end(bm::PK_COL, st);
 		return rc;
 	}
 	rc = bm::pass_y(m->Ny, -1, m->S, m->Sx, nlines, m->Sp, m->NC, m->ntl, m->ncu, st, fy);

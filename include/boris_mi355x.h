@@ -412,7 +412,8 @@ int bm_adj_batch_backward(int count, const bm_adj_t* h, float* const* gMs_out, d
  * 4 x-C2R pass, 5 2D y pass with kernel multiply, 6 field + RK stage (no demag),
  * 7 RKDP54 advance (no demag), 8 fused row kernel (x-C2R of H_demag + field + RK stage +
  * x-R2C of the stage's output M), 9 x-R2C pass fused with the RKDP54 advance,
- * 10 multilayer kernel product.
+ * 10 multilayer kernel product, 11 column pass (both y passes and the z pass, 2D or
+ * multilayer product between them as one kernel).
  * Not thread safe; meant for benchmarks. */
 int bm_prof_begin(int max_launches);
 int bm_prof_end(void);

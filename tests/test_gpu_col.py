@@ -2,11 +2,13 @@
 at the fewest and most planes or layers of each, open and periodic y, against the FP64 oracle (the
 field's parity bar, 1e-6 relative L2), and against the separate passes, whose arithmetic it repeats
 (FP32 rounding: 5e-7; a field evaluation's own error is below 2e-7)."""
+import ctypes as C
+
 import numpy as np
 import pytest
 import torch
 
-from boris2_amd import api
+from boris2_amd import _lib, api
 import oracle_lib as O
 
 pytestmark = pytest.mark.gpu
@@ -85,4 +87,27 @@ def test_layers_first_and_last_column_as_one(gpu, nx, ny, L):
     d = api.MultiLayerDemag(nx, ny, 4e-9, 4e-9, [4e-9] * L, z0)
     ref = O.OracleMLayer(nx, ny, 4e-9, 4e-9, np.full(L, 4e-9), np.array(z0))(M0.astype(np.float64))
     assert rel(d.convolute(torch.from_numpy(M0).cuda()).cpu().numpy().astype(np.float64), np.asarray(ref).reshape(-1, 3)) <= 1e-6
+    d.close()
+
+
+@pytest.mark.parametrize("n", [(64, 64, 1), (64, 32, 4), (32, 32, -3)])
+def test_column_pass_is_timed_as_itself(gpu, n):
+    """Launch timing counts the column kernel (kind 11) and no y, z, 2D or product pass; n[2] < 0: layers."""
+    L = _lib.load()
+    if n[2] < 0:
+        d = api.MultiLayerDemag(n[0], n[1], 4e-9, 4e-9, [4e-9] * 3, [8e-9 * l for l in range(3)])
+    else:
+        d = api.Demag(n, H)
+    M = torch.ones((n[0] * n[1] * abs(n[2]), 3), device="cuda")
+    _lib.check(L.bm_prof_begin(16))
+    d.convolute(M)
+    torch.cuda.synchronize()
+    _lib.check(L.bm_prof_end())
+    count = {}
+    for k, name in enumerate(_lib.PROF_KINDS):
+        c = C.c_longlong()
+        _lib.check(L.bm_prof_query(k, C.byref(c), None, None, None))
+        if c.value:
+            count[name] = c.value
+    assert count == {"fwd_x_r2c": 1, "column_pass": 1, "inv_x_c2r": 1}
     d.close()
