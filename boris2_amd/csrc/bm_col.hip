@@ -349,10 +349,9 @@ template <int NY, int V> bool col_items(int P)
 
 // kind: N.z (3D, open z: 4 to 32), 1 (2D) or 0 (layers).  Where the lines fit, against the separate
 // passes (field of a mesh, separate -> column): 64x64x1 14.7 -> 12.0 us, 128x128x4 25.3 -> 17.2,
-// 128x128x8 31.0 -> 24.5, 512x512x4 104 -> 88, layers 128x128x8 54.1 -> 32.5; 512x512x1 37.9 -> 39.1
-// and 256x256x8 60.0 -> 59.2, where one or two columns per compute unit leave its loads, transforms
-// and stores one after another.  Not for radix-3 lengths with N.z >= 16 beyond one column per
-// compute unit (256x192x8 52 -> 62, 512x192x8 88 -> 95: the longer schedules of 12 values per thread).
+// 128x128x8 31.0 -> 24.5, 512x512x4 104 -> 88, layers 128x128x8 54.1 -> 32.5, 256x256x8 60.0 -> 59.2.
+// Not for radix-3 lengths with N.z >= 16 beyond one column per compute unit (256x192x8 52 -> 62,
+// 512x192x8 88 -> 95: the longer schedules of 12 values per thread).
 bool bm::col_ok(int Ny, int kind, int P, int NC, int ncu)
 {
 	if (kind > 1 && kind != 4 && kind != 8 && kind != 16 && kind != 32) return false;

@@ -1020,9 +1020,16 @@ bool yzy_ok(const bm_demag_s* d)
 
 // The column pass serves this mesh (open z) and is the better one: from N.y = 1024 with N.z = 4 the
 // thin-mesh pass, which keeps both planes in registers, is faster (512x512x2 61.0 -> 57.0 us,
-// 768x512x2 93 -> 81; 1024x256x2 57.5 -> 58.8, 256x256x2 23.8 -> 26.7).
-bool use_col(const bm_demag_s* d)
+// 768x512x2 93 -> 81; 1024x256x2 57.5 -> 58.8, 256x256x2 23.8 -> 26.7).  Nor, for a mesh on its own,
+// 2D lines of 1024 with more than two and at most four columns per compute unit: a compute unit runs
+// two of these columns at a time (three waves each, two waves per SIMD by registers), but four in
+// the 2D y pass (two workgroups of two, one wave per SIMD), which then needs one round where the
+// column pass needs two (middle of 512x512x1 18.1 us against 20.9, 768x512x1 21.4 / 24.7, periodic
+// 1024x1024x1 22.1 / 24.0; with fewer columns 384x512x1 17.8 / 15.7, with more, as a batch of such
+// films has them, 1024x512x1 34.0 / 30.0 and 2048x512x1 49.7 / 45.9).
+bool use_col(const bm_demag_s* d, bool alone)
 {
+	if (alone && d->is2d && d->Ny == 1024 && d->NC > 2 * d->ncu && d->NC <= 4 * d->ncu) return false;
 	if (!d->yzy || d->full[2] || pass_tune().y_radix || pass_tune().y_percu || pass_tune().z_radix || pass_tune().z_percu) return false;
 	if (yzy_ok(d) && (d->yzy == 2 || d->Ny >= 1024)) return false;
 	return col_ok(d->Ny, d->Nz, d->nz, d->NC, d->ncu);
@@ -1209,7 +1216,7 @@ int bm::demag_mid(bm_demag_s* d, hipStream_t st)
 {
 	const int nlines = 3 * d->nz * d->NC;
 	int rc;
-	if (use_col(d)) {
+	if (use_col(d, true)) {
 		prof_mark_begin(PK_COL, st);
 		rc = launch_col(d->Ny, d->Nz, d->full[1], d->Sx, d->K, nullptr, d->nz, d->NC, d->NYH, d->ntl, d->full[1] ? d->Ny : d->ny, 0, d->ncu, st);
 		prof_mark_end(PK_COL, st);
@@ -1763,7 +1770,7 @@ int bm::batch_y2d(int Ny, bool full, LaunchShape sh, const PassBatch* h_tab, con
 }
 
 bool bm::demag_yzy(const bm_demag_s* d) { return yzy_ok(d); }
-bool bm::demag_col(const bm_demag_s* d) { return use_col(d); }
+bool bm::demag_col(const bm_demag_s* d) { return use_col(d, false); }
 
 int bm::batch_yzy(int Ny, int Nz, LaunchShape sh, const PassBatch* h_tab, const PassBatch* d_tab, int nb, int ncu, hipStream_t st)
 {

@@ -190,7 +190,7 @@ int batch_y2d(int Ny, bool full, LaunchShape sh, const PassBatch* h_tab, const P
 // thin meshes (N.z 4 or 8, open y and z, a power-of-two N.y with a fitting schedule): the y, z,
 // y passes as one kernel that never writes the full spectra; demag_yzy: the handle takes it
 bool demag_yzy(const bm_demag_s* d);
-// the handle's middle passes run as the column pass
+// the handle's middle passes run as the column pass in a batch
 bool demag_col(const bm_demag_s* d);
 int batch_yzy(int Ny, int Nz, LaunchShape sh, const PassBatch* h_tab, const PassBatch* d_tab, int nb, int ncu, hipStream_t st);
 }

@@ -111,3 +111,27 @@ def test_column_pass_is_timed_as_itself(gpu, n):
             count[name] = c.value
     assert count == {"fwd_x_r2c": 1, "column_pass": 1, "inv_x_c2r": 1}
     d.close()
+
+
+@pytest.mark.parametrize("n,pbc,col", [((384, 512, 1), (0, 0, 0), 1), ((400, 400, 1), (0, 0, 0), 0), ((768, 385, 1), (0, 0, 0), 0), ((1024, 400, 1), (0, 0, 0), 1),
+                                       ((1024, 1024, 1), (2, 2, 0), 0)])
+def test_2d_lines_of_1024(gpu, n, pbc, col):
+    """Between two and four columns per compute unit these take the 2D y pass, else the column kernel;
+    either way the field is the oracle's."""
+    L = _lib.load()
+    ncu = torch.cuda.get_device_properties(0).multi_processor_count
+    if ncu != 256:
+        pytest.skip("the column counts are chosen around 256 compute units")
+    M0 = api.random_magnetisation(n[0] * n[1], 8e5, 2).astype(np.float32)
+    M = torch.from_numpy(M0).cuda()
+    d = api.Demag(n, H, pbc)
+    _lib.check(L.bm_prof_begin(16))
+    got = d.convolute(M).cpu().numpy().astype(np.float64)
+    _lib.check(L.bm_prof_end())
+    c = C.c_longlong()
+    _lib.check(L.bm_prof_query(_lib.PROF_KINDS.index("column_pass"), C.byref(c), None, None, None))
+    N = d.info()[0]
+    assert N[1] == 1024 and c.value == col
+    ref = O.OracleDemag(n, H, pbc=pbc)(M0.astype(np.float64))
+    assert rel(got, ref) <= 1e-6
+    d.close()
