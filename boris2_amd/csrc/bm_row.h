@@ -230,6 +230,14 @@ inline int row_grid(int nwork, int ncu)
 	return ((g + 7) / 8) * 8;
 }
 
+template <int HX, int METHOD, int STEP, bool R2C, int NG>
+void launch_rows_t(const RowGeom& d, const StageArgs& a, int nwork, int ns, float scale, hipStream_t st)
+{
+	const dim3 g((nwork + 7) / 8 * 8), b(XSplit<HX, NG>::BS);
+	if (a.layered) hipLaunchKernelGGL((k_rows<HX, METHOD, STEP, R2C, true, NG>), g, b, 0, st, a, d.Sx, d.ntl, ns, scale);
+	else hipLaunchKernelGGL((k_rows<HX, METHOD, STEP, R2C, false, NG>), g, b, 0, st, a, d.Sx, d.ntl, ns, scale);
+}
+
 template <int METHOD, int STEP, bool R2C>
 int launch_row_t(const RowGeom& d, const StageArgs& a, float scale, hipStream_t st)
 {
@@ -243,9 +251,8 @@ int launch_row_t(const RowGeom& d, const StageArgs& a, float scale, hipStream_t 
 #define C_(V_) case V_: { \
 	if constexpr (xs_ok<V_>()) if (xs_few_rows(V_, d.ny, d.nz, d.ncu, true)) { \
 		const int ns = (d.ny + XSplit<V_>::RP - 1) / XSplit<V_>::RP, g = d.nz * ns; \
-		const dim3 gd((g + 7) / 8 * 8), bd(a.layered ? XSplit<V_, xs_groups<V_, true>()>::BS : XSplit<V_, xs_groups<V_>()>::BS); \
-		if (a.layered) hipLaunchKernelGGL((k_rows<V_, METHOD, STEP, R2C, true>), gd, bd, 0, st, a, d.Sx, d.ntl, ns, scale); \
-		else hipLaunchKernelGGL((k_rows<V_, METHOD, STEP, R2C, false>), gd, bd, 0, st, a, d.Sx, d.ntl, ns, scale); \
+		if constexpr (xs_row_both<V_>()) if (xs_row_four(g, d.ncu)) { launch_rows_t<V_, METHOD, STEP, R2C, 4>(d, a, g, ns, scale, st); return BM_OK; } \
+		launch_rows_t<V_, METHOD, STEP, R2C, xs_groups<V_>()>(d, a, g, ns, scale, st); \
 		return BM_OK; \
 	} \
 	if constexpr (!xs_row_only<V_>()) { \

@@ -31,13 +31,20 @@ template <int HX> constexpr bool xs_row_only() { return xs_ok<HX>() && Plan<HX>:
 // wave groups of the kernels with much per-cell work: with 8 values per thread the 32 W E cell pairs of
 // a workgroup are a third more than three groups, so rows of 16 lanes or fewer take a fourth wave for
 // the per-cell work only (one round instead of two: 128x64 film RK4 step 48.1 -> 46.9 us, ten 128x64
-// layers 105 -> 101).  At 256 cells per row (32 lanes) it pays for layer stacks, which are small (LAY;
-// RK4 step of three 256x256 layers 116 -> 111 us), and costs larger meshes more (256x256x8, three
-// RKDP54 steps 1024 -> 1064 us).
-template <int HX, bool LAY = false> constexpr int xs_groups()
+// layers 105 -> 101).
+template <int HX> constexpr int xs_groups()
 {
-	return xs_waves<HX>() == 1 && Plan<HX>::E == 8 && plan_T<HX>() <= (LAY ? 32 : 16) ? 4 : 3;
+	return xs_waves<HX>() == 1 && Plan<HX>::E == 8 && plan_T<HX>() <= 16 ? 4 : 3;
 }
+// The row kernel at 32 lanes (256 cells per row) has both forms.  Its registers leave three waves per
+// SIMD, so a compute unit holds four workgroups of three waves or three of four: the fourth wave
+// pays (RK4 steps of 256x256 cells by 1, 3, 6 planes 65.6 -> 63.1, 125.5 -> 121.4, 186.1 -> 180.5 us, of
+// 3 layers 123.0 -> 117.4) but where the workgroups are more than three and at most four per compute
+// unit, one round without it and two with (256x256 by 7 and 8 planes 205.9 -> 212.9, 208.7 -> 216.0, of
+// 8 layers 298 -> 305); from the second round on it pays again (9, 12, 24 planes 303 -> 293, 339 -> 330,
+// 607 -> 590).
+template <int HX> constexpr bool xs_row_both() { return xs_waves<HX>() == 1 && Plan<HX>::E == 8 && plan_T<HX>() == 32; }
+inline bool xs_row_four(int workgroups, int ncu) { return workgroups <= 3 * ncu || workgroups > 4 * ncu; }
 
 template <int HX, int NG = 3> struct XSplit {
 	static constexpr int W = xs_waves<HX>(), WT = 64 * W, E = Plan<HX>::E, T = plan_T<HX>();
@@ -227,10 +234,11 @@ __global__ void __launch_bounds__((XSplit<HX, xs_inv_groups<HX, MODE>()>::BS)) k
 
 // The fused row kernel (k_row) in this form; LAY: a layer stack (the planes are the layers), a form of
 // its own because the per-layer values cost plain meshes 3 % (RK4 step of a 128x64 film 47.8 -> 49.5 us).
-template <int HX, int METHOD, int STEP, bool R2C, bool LAY>
-__global__ void __launch_bounds__((XSplit<HX, xs_groups<HX, LAY>()>::BS)) k_rows(StageArgs a, float2* Sx, int ntl, int ntiles, float scale)
+// NG: its wave groups.
+template <int HX, int METHOD, int STEP, bool R2C, bool LAY, int NG>
+__global__ void __launch_bounds__((XSplit<HX, NG>::BS)) k_rows(StageArgs a, float2* Sx, int ntl, int ntiles, float scale)
 {
-	using X = XSplit<HX, xs_groups<HX, LAY>()>;
+	using X = XSplit<HX, NG>;
 	__shared__ C2<float> tile[3 * X::RP * X::P];
 	X x; x.init(tile);
 	constexpr int EL = X::E / 2, NP = HX / 2;

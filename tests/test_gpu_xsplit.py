@@ -122,3 +122,15 @@ def test_stack_field_function_may_use_the_stacks_handle(gpu):
         out.append(s.M.clone())
         s.close()
     assert torch.equal(out[0], out[1])
+
+
+# 256 cells per row: workgroups (two rows each) up to three per compute unit, from there to four (no
+# fourth wave), and more
+@pytest.mark.parametrize("ny,nz", [(127, 12), (220, 7), (128, 16), (129, 16)])
+@pytest.mark.parametrize("method", [api.BM_EVAL_RK4, api.BM_EVAL_RKDP54])
+def test_steps_around_the_fourth_wave(gpu, ny, nz, method):
+    test_steps(gpu, (256, ny, nz), method)
+
+
+def test_layer_stack_without_the_fourth_wave(gpu, monkeypatch):
+    test_layer_stack_rows_match_the_separate_passes(gpu, monkeypatch, 256, 192, [0, 0, 1, 1, 2, 3, 4, 4, 5], api.BM_EVAL_RK4)
