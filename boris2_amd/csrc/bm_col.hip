@@ -33,15 +33,16 @@ struct ColArgs {
 	float2* Sx; const float* K; const int* kidx;
 	int P, NC, NYH, ntl, nyd, lpk, tr;
 	const ColBatch* bt;     // batched: one mesh or stack per grid row
-	int ncu;                // compute units
+	int ncu;                // compute units (for the launchers)
 };
 
-// The columns kx = 0 and kx = N.x / 2 hold real values: in the z form from N.z = 16, whose
-// workgroups fill a compute unit each, the first workgroup takes both as one complex line (first + i second) where a column more
+// The columns kx = 0 and kx = N.x / 2 hold real values: in the z form of one mesh from N.z = 16 (PACK),
+// whose workgroups fill a compute unit each, the first workgroup takes both as one complex line (first + i second) where a column more
 // than a multiple of the compute units would cost a round of its own (RK4 steps: 256x256x8, 257
 // columns on 256 units, 235 -> 212 us, 256x128x16 242 -> 228, 512x256x8 389 -> 369).  A real line's transform is X(-ky) = conj X(ky), so the two spectra come apart
 // (and together) within the pair (ky, -ky): both are worked on for ky = 0 .. N.y / 2, column 0's
-// results at ky and the other's at N.y - ky, both in one value at ky = 0 and N.y / 2.
+// results at ky and the other's at N.y - ky, both in one value at ky = 0 and N.y / 2.  Not in batches,
+// whose meshes share the rounds: a mesh there computes the same bits whatever runs beside it.
 __device__ __forceinline__ C2<float> pair_get(const C2<float>* line, int NY, int ky, int col)
 {
 	const C2<float> a = line[ky], b = line[ky ? NY - ky : 0];
@@ -71,7 +72,7 @@ __device__ __forceinline__ C2<float> lane_xor1(C2<float> v) { return lane_quad<0
 __device__ __forceinline__ C2<float> lane_xor2(C2<float> v) { return lane_quad<0x4E>(v); }   // lanes 2 3 0 1
 
 // The z transform of N.z points on M adjacent lanes (up to 8 values each), the plan's stages with
-// the exchange between them through lane swaps instead of LDS: the same bits as the z pass's.
+// the exchange between them through lane swaps instead of LDS.
 template <int NZ> struct ZLanes {
 	static constexpr int M = plan_T<NZ>(), R1 = Plan<NZ>::S > 1 ? Plan<NZ>::R[Plan<NZ>::S - 1] : 1;
 	static_assert(M == R1 && M <= 4 && Plan<NZ>::S <= 2, "one radix-8 stage, then one over the lanes");
@@ -121,7 +122,7 @@ template <int NZ> struct ZLanes {
 	}
 };
 
-__device__ __host__ __forceinline__ bool col_packed(int lpk, int NC, int ncu) { return lpk == 1 && NC > ncu && (NC - 1) % ncu == 0; }
+inline bool col_packed(int lpk, int NC, int ncu) { return lpk == 1 && NC > ncu && (NC - 1) % ncu == 0; }
 
 template <int NY, int KIND, int NZ, bool FULL, bool PACK>
 __global__ void __launch_bounds__((col_threads<KIND, NZ>()), (KIND == COL_LAYERS && NY < 1024 ? 4 : 1)) k_col(ColArgs a)
@@ -135,8 +136,8 @@ __global__ void __launch_bounds__((col_threads<KIND, NZ>()), (KIND == COL_LAYERS
 	}
 	const int lane = threadIdx.x & 63, t = lane % T, sub = lane / T, stride = (blockDim.x >> 6) * LW;
 	const int P = KIND == COL_2D ? 1 : a.P, lpk = a.lpk, nl = 3 * P * lpk, kx0 = blockIdx.x * lpk;
-	const bool packed = PACK && col_packed(lpk, a.NC, a.ncu), both = PACK && packed && blockIdx.x == 0;
-	if (kx0 >= a.NC - (packed ? 1 : 0)) return;                 // uniform over the block
+	const bool both = PACK && blockIdx.x == 0;
+	if (kx0 >= a.NC) return;                                   // uniform over the block
 	Twiddles<NY, float> tw; tw.init(t);
 
 	// lines li = (c P + z) lpk + column: the next round's values are loaded while this one's are
@@ -320,15 +321,15 @@ template <int NY, int KIND, int NZ> ColShape col_shape(int P)
 template <int NY, int KIND, int NZ, bool FULL, bool PACK = false>
 int launch_col_t(const ColArgs& in, int nb, hipStream_t st)
 {
-	// the z form with one workgroup per compute unit: columns 0 and N.x / 2 as one
+	// the z form of one mesh with one workgroup per compute unit: columns 0 and N.x / 2 as one
 	if constexpr (KIND == COL_Z && NZ >= 16 && !PACK)
-		if (in.bt ? in.NC > in.ncu : col_packed(col_shape<NY, KIND, NZ>(in.P).lpk, in.NC, in.ncu)) return launch_col_t<NY, KIND, NZ, FULL, true>(in, nb, st);
+		if (!in.bt && col_packed(col_shape<NY, KIND, NZ>(in.P).lpk, in.NC, in.ncu)) return launch_col_t<NY, KIND, NZ, FULL, true>(in, nb, st);
 	const ColShape s = col_shape<NY, KIND, NZ>(in.P);
 	ColArgs a = in;
 	a.lpk = s.lpk;
 	if (s.lds > 65536)
 		BM_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(&k_col<NY, KIND, NZ, FULL, PACK>), hipFuncAttributeMaxDynamicSharedMemorySize, (int)s.lds));
-	hipLaunchKernelGGL((k_col<NY, KIND, NZ, FULL, PACK>), dim3((a.NC - (PACK && !a.bt) + s.lpk - 1) / s.lpk, nb), dim3(s.threads), s.lds, st, a);
+	hipLaunchKernelGGL((k_col<NY, KIND, NZ, FULL, PACK>), dim3((a.NC - PACK + s.lpk - 1) / s.lpk, nb), dim3(s.threads), s.lds, st, a);
 	return BM_OK;
 }
 
