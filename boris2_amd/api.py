@@ -471,8 +471,8 @@ class BatchSolver:
     layers: None, or per mesh None or dict(hz=..., z0=..., Ms=None, A=None, alpha=None,
     K1=None) making that mesh's n[2] planes a layer stack (as LayerStackSolver).
     autotune: False, True (launch shapes timed before the first step; results unchanged bit
-    for bit) or "radix" (the FFT passes' radix schedules timed too; results within FP32
-    rounding of the default schedules).  pbc: None, or per mesh None or (px, py, pz) periodic
+    for bit) or "radix" (the FFT passes' radix schedules timed too, and the column kernel against the
+    separate passes; results within FP32 rounding of the default schedules).  pbc: None, or per mesh None or (px, py, pz) periodic
     images (as FMSolver's pbc)."""
 
     def __init__(self, method: int, meshes, M0=None, use_graph: bool = True, layers=None, autotune=False, pbc=None):
@@ -530,7 +530,8 @@ class BatchSolver:
 
     def set_schedule(self, pass_: str, size: int, f: int = 0, per_cu: int = 0, radix: int = 0) -> None:
         """Pin one pass-size group's launch shape and radix schedule (pass_: x_fwd, x_inv, y_fwd,
-        y_inv, z, y2d, ml_mult), replacing any pending autotuning."""
+        y_inv, z, y2d, yzy4, yzy8, ml_mult; or a column group, col_2d, col_ml, col_z<N.z> by N.y: f = 1
+        the column kernel, 2 the separate passes), replacing any pending autotuning."""
         check(self.L.bm_batch_set_schedule(self.handle, pass_.encode(), int(size), int(f), int(per_cu), int(radix)))
 
     def apply_report(self, lines) -> None:

@@ -97,9 +97,10 @@ struct bm_batch_s {
 	std::vector<Tab<PassBatch>> inv, ty, tz, ty2;
 	std::vector<Tab<MlBatch>> tml;
 	std::vector<Tab<PassBatch>> tyz[2];
-	// meshes whose middle passes run as the column pass (bm_col.hip), by N.y, kind and periodic y:
-	// those it serves whose y, z, 2D y, fused and product groups all have their default shapes
-	struct ColGroup { int Ny, kind; bool full; Tab<ColBatch> t; };
+	// the meshes that the column pass (bm_col.hip) can serve, by N.y, periodic y and kind.  The factor of
+	// g.sh[0] chooses for the group: 1 the column pass, 2 the separate passes, 0 the column pass
+	// except for meshes with a y, z or 2D y pass pinned to another radix schedule.
+	struct ColGroup { Group g; int kind; Tab<ColBatch> t; };
 	std::vector<ColGroup> gcol;
 	bool no_col = false;                   // while the autotuner times the separate passes
 	Tab<StageArgs> stage[2];               // [input parity]
@@ -295,6 +296,12 @@ __global__ void k_rkdp_end(BatchCtl* ctl, int nb)
 	if (c.iteration >= c.target) c.active = 0;
 }
 
+void add_col(bm_batch_s* o, int Ny, bool full, int kind, int b)
+{
+	for (auto& c : o->gcol) if (c.g.size == Ny && c.g.full == full && c.kind == kind) { c.g.meshes.push_back(b); return; }
+	o->gcol.push_back({ Group{ Ny, full, { b } }, kind, {} });
+}
+
 // Group the meshes by pass size.
 void build_groups(bm_batch_s* o)
 {
@@ -305,10 +312,12 @@ void build_groups(bm_batch_s* o)
 			add_to(o->gx, o->nx[b], false, b);
 			add_to(o->gy, v.Ny, false, b);
 			add_to(o->gml, v.L, false, b);
+			if (col_ok(v.Ny, 0, v.L, v.NC, o->ncu)) add_col(o, v.Ny, false, 0, b);
 			continue;
 		}
 		const bm_demag_s* d = o->dm[b];
 		if (!d) continue;
+		if (demag_col(d)) add_col(o, d->Ny, d->full[1], d->Nz, b);
 		// a periodic x pass transforms rows of N.x = nx cells as nx/2-point complex FFTs
 		const bool fx = d->pbc[0] > 0, fy = d->pbc[1] > 0, fz = d->pbc[2] > 0;
 		add_to(o->gx, fx ? d->Nx / 2 : o->nx[b], fx, b);
@@ -319,36 +328,31 @@ void build_groups(bm_batch_s* o)
 }
 
 // Build every table on the host (x tables depend on the groups' tile factors) and upload
-// them in one allocation, replacing earlier tables.
-int build_tables(bm_batch_s* o)
+// them in one allocation, replacing earlier tables.  only: the middle passes of these meshes alone
+// (while the autotuner compares their two forms).
+int build_tables(bm_batch_s* o, const std::vector<int>* only = nullptr)
 {
 	const int nb = o->nb;
 	if (o->dev_tables) { (void)hipFree(o->dev_tables); o->dev_tables = nullptr; }
-	std::vector<char> col((size_t)nb, 0);
-	o->gcol.clear();
-	{
-		std::vector<char> pinned((size_t)nb, 0);
-		for (const std::vector<Group>* gs : { &o->gy, &o->gz, &o->gy2, &o->gml, &o->gyz[0], &o->gyz[1] })
-			for (const Group& G : *gs)
-				for (int q = 0; q < 2; q++) if (G.sh[q].f || G.sh[q].per_cu || G.sh[q].radix) for (int b : G.meshes) pinned[(size_t)b] = 1;
-		for (int b = 0; b < nb; b++) {
-			if (o->no_col || pinned[(size_t)b] || (!o->ml[b] && !o->dm[b])) continue;
-			int Ny, kind; bool full = false; ColBatch t;
+	// col: the mesh has no separate middle passes
+	std::vector<char> col((size_t)nb, only ? 1 : 0), pinned((size_t)nb, 0);
+	if (only) for (int b : *only) col[(size_t)b] = 0;
+	for (const std::vector<Group>* gs : { &o->gy, &o->gz, &o->gy2 })
+		for (const Group& G : *gs) if (G.sh[0].radix || G.sh[1].radix) for (int b : G.meshes) pinned[(size_t)b] = 1;
+	for (auto& c : o->gcol) {
+		c.t.h.clear();
+		const int f = c.g.sh[0].f;
+		for (int b : c.g.meshes) {
+			if (o->no_col || col[(size_t)b] || f == 2 || (f == 0 && pinned[(size_t)b])) continue;
 			if (o->ml[b]) {
 				const MlView v = mlayer_view(o->ml[b]);
-				if (!col_ok(v.Ny, 0, v.L, v.NC, o->ncu)) continue;
-				Ny = v.Ny; kind = 0; t = ColBatch{ v.Sx, v.K, v.kcol, v.L, v.NC, v.NYH, v.ntl, v.ny };
+				c.t.h.push_back(ColBatch{ v.Sx, v.K, v.kcol, v.L, v.NC, v.NYH, v.ntl, v.ny });
 			}
 			else {
 				const bm_demag_s* d = o->dm[b];
-				if (!demag_col(d)) continue;
-				Ny = d->Ny; kind = d->Nz; full = d->full[1]; t = ColBatch{ d->Sx, d->K, nullptr, d->nz, d->NC, d->NYH, d->ntl, full ? d->Ny : d->ny };
+				c.t.h.push_back(ColBatch{ d->Sx, d->K, nullptr, d->nz, d->NC, d->NYH, d->ntl, d->full[1] ? d->Ny : d->ny });
 			}
 			col[(size_t)b] = 1;
-			bm_batch_s::ColGroup* g = nullptr;
-			for (auto& q : o->gcol) if (q.Ny == Ny && q.kind == kind && q.full == full) g = &q;
-			if (!g) { o->gcol.push_back({ Ny, kind, full, {} }); g = &o->gcol.back(); }
-			g->t.h.push_back(t);
 		}
 	}
 	for (int par = 0; par < 2; par++) o->fwd[par].assign(o->gx.size(), Tab<FwdArgs>());
@@ -443,7 +447,7 @@ int build_tables(bm_batch_s* o)
 	std::vector<size_t> at_yz[2];
 	for (int q = 0; q < 2; q++) for (auto& t : o->tyz[q]) at_yz[q].push_back(place(t));
 	std::vector<size_t> at_col;
-	for (auto& g : o->gcol) at_col.push_back(place(g.t));
+	for (auto& c : o->gcol) at_col.push_back(place(c.t));
 	const size_t at_s0 = place(o->stage[0]), at_s1 = place(o->stage[1]), at_ch = place(o->choff);
 	if (hipMalloc(&o->dev_tables, std::max<size_t>(bytes, 256)) != hipSuccess) return fail(BM_ERR_NOMEM, "batch tables");
 	o->dev_bytes = bytes;
@@ -504,14 +508,21 @@ template <class T> std::vector<size_t> live(const std::vector<Tab<T>>& tabs)
 	return r;
 }
 
+int launch_col_group(bm_batch_s* o, bm_batch_s::ColGroup& c, hipStream_t st)
+{
+	return batch_col(c.g.size, c.kind, c.g.full, c.t.h.data(), c.t.d, (int)c.t.h.size(), o->ncu, st);
+}
+
 // The middle passes of every mesh: first the meshes with one kernel for them (column, 2D y and
 // thin-mesh passes, all groups side by side), then the chain of separate passes.
 int middle_all(bm_batch_s* o, hipStream_t st)
 {
 	const std::vector<size_t> l2 = live(o->ty2), l4 = live(o->tyz[0]), l8 = live(o->tyz[1]), ly = live(o->ty), lz = live(o->tz), lm = live(o->tml);
-	const size_t nc = o->gcol.size();
+	std::vector<size_t> lc;
+	for (size_t q = 0; q < o->gcol.size(); q++) if (!o->gcol[q].t.h.empty()) lc.push_back(q);
+	const size_t nc = lc.size();
 	int rc = fan(o, nc + l2.size() + l4.size() + l8.size(), st, [&](size_t q, hipStream_t s) {
-		if (q < nc) { auto& g = o->gcol[q]; return batch_col(g.Ny, g.kind, g.full, g.t.h.data(), g.t.d, (int)g.t.h.size(), o->ncu, s); }
+		if (q < nc) return launch_col_group(o, o->gcol[lc[q]], s);
 		if ((q -= nc) < l2.size()) {
 			const size_t g = l2[q];
 			return batch_y2d(o->gy2[g].size, o->gy2[g].full, o->gy2[g].sh[0], o->ty2[g].h.data(), o->ty2[g].d, (int)o->ty2[g].h.size(), o->ncu, s);
@@ -553,8 +564,8 @@ int eval_all(bm_batch_s* o, int step, int par, hipStream_t st)
 // launches after a warm-up, HIP events) on the group's real tables and keep the fastest.
 // Candidates: x passes the default, tile factor {1, 2} x workgroups per CU {1, 2, 4}, and the
 // half-height tile at {2, 4, 8} per CU where the row length has one; y passes {4, 8, 16};
-// z pass {1, 2, 4}; 2D y pass {4, 8, 16}; multilayer product {4, 8, 16}.  Then the middle passes
-// as a whole, tuned, against their default shapes (with which meshes take the column pass).  Only the FFT passes
+// z pass {1, 2, 4}; 2D y pass {4, 8, 16}; multilayer product {4, 8, 16}.  Then, with radix tuning, for
+// every column group its meshes' column pass against their separate passes.  Only the FFT passes
 // run (their inputs are recomputed from M by every evaluation), so the state is untouched.
 int autotune(bm_batch_s* o, hipStream_t st)
 {
@@ -610,39 +621,57 @@ int autotune(bm_batch_s* o, hipStream_t st)
 		pick(G, 0, cands, true, [&] { return batch_fwd_x(G.size, G.full, G.sh[0], o->fwd[0][g].h.data(), o->fwd[0][g].d, (int)o->fwd[0][g].h.size(), o->ncu, st); });
 		if (!rc) pick(G, 1, cands, true, [&] { return batch_inv_x_planar(G.size, G.full, G.sh[1], o->inv[g].h.data(), o->inv[g].d, (int)o->inv[g].h.size(), o->ncu, st); });
 	}
-	for (size_t g = 0; g < o->gy.size() && !rc; g++) {
-		Group& G = o->gy[g];
-		for (int slot = 0; slot < 2; slot++)
-			pick(G, slot, radices(cy, G.size, G.full), false, [&] { return batch_y(G.size, G.full, slot ? 1 : -1, G.sh[slot], o->ty[g].h.data(), o->ty[g].d, (int)o->ty[g].h.size(), o->ncu, st); });
-	}
-	for (size_t g = 0; g < o->gz.size() && !rc; g++) {
-		Group& G = o->gz[g];
-		pick(G, 0, radices(cz, G.size, G.full), false, [&] { return batch_z(G.size, G.full, G.sh[0], o->tz[g].h.data(), o->tz[g].d, (int)o->tz[g].h.size(), o->ncu, st); });
-	}
-	for (size_t g = 0; g < o->gy2.size() && !rc; g++) {
-		Group& G = o->gy2[g];
-		pick(G, 0, radices(cy, G.size, G.full), false, [&] { return batch_y2d(G.size, G.full, G.sh[0], o->ty2[g].h.data(), o->ty2[g].d, (int)o->ty2[g].h.size(), o->ncu, st); });
-	}
-	for (size_t g = 0; g < o->gml.size() && !rc; g++) {
-		Group& G = o->gml[g];
-		pick(G, 0, cy, false, [&] { return batch_ml_mult(G.size, G.sh[0], o->tml[g].h.data(), o->tml[g].d, (int)o->tml[g].h.size(), o->ncu, st); });
-	}
-	for (int q = 0; q < 2 && !rc; q++)
-		for (size_t g = 0; g < o->gyz[q].size() && !rc; g++) {
-			Group& G = o->gyz[q][g];
-			pick(G, 0, cy, false, [&] { return batch_yzy(G.size, q ? 8 : 4, G.sh[0], o->tyz[q][g].h.data(), o->tyz[q][g].d, (int)o->tyz[q][g].h.size(), o->ncu, st); });
+	// the separate middle passes; left: only those that some of their meshes have left
+	auto tune_middle = [&](bool left) {
+		auto skip = [&](const Group& G, size_t meshes) { return rc || meshes == 0 || (left && meshes == G.meshes.size()); };
+		for (size_t g = 0; g < o->gy.size(); g++) {
+			Group& G = o->gy[g];
+			if (skip(G, o->ty[g].h.size())) continue;
+			for (int slot = 0; slot < 2; slot++)
+				pick(G, slot, radices(cy, G.size, G.full), false, [&] { return batch_y(G.size, G.full, slot ? 1 : -1, G.sh[slot], o->ty[g].h.data(), o->ty[g].d, (int)o->ty[g].h.size(), o->ncu, st); });
 		}
-	if (!rc) {
-		const double tuned = timed([&] { return middle_all(o, st); });
+		for (size_t g = 0; g < o->gz.size(); g++) {
+			Group& G = o->gz[g];
+			if (skip(G, o->tz[g].h.size())) continue;
+			pick(G, 0, radices(cz, G.size, G.full), false, [&] { return batch_z(G.size, G.full, G.sh[0], o->tz[g].h.data(), o->tz[g].d, (int)o->tz[g].h.size(), o->ncu, st); });
+		}
+		for (size_t g = 0; g < o->gy2.size(); g++) {
+			Group& G = o->gy2[g];
+			if (skip(G, o->ty2[g].h.size())) continue;
+			pick(G, 0, radices(cy, G.size, G.full), false, [&] { return batch_y2d(G.size, G.full, G.sh[0], o->ty2[g].h.data(), o->ty2[g].d, (int)o->ty2[g].h.size(), o->ncu, st); });
+		}
+		for (size_t g = 0; g < o->gml.size(); g++) {
+			Group& G = o->gml[g];
+			if (skip(G, o->tml[g].h.size())) continue;
+			pick(G, 0, cy, false, [&] { return batch_ml_mult(G.size, G.sh[0], o->tml[g].h.data(), o->tml[g].d, (int)o->tml[g].h.size(), o->ncu, st); });
+		}
+		for (int q = 0; q < 2; q++)
+			for (size_t g = 0; g < o->gyz[q].size(); g++) {
+				Group& G = o->gyz[q][g];
+				if (skip(G, o->tyz[q][g].h.size())) continue;
+				pick(G, 0, cy, false, [&] { return batch_yzy(G.size, q ? 8 : 4, G.sh[0], o->tyz[q][g].h.data(), o->tyz[q][g].d, (int)o->tyz[q][g].h.size(), o->ncu, st); });
+			}
+	};
+	tune_middle(false);
+	// Each column group's time and, with radix tuning, its meshes' column pass against their separate
+	// passes as just tuned.  Without it the forms stay, as they round differently (the compiler's
+	// contractions differ, the thin-mesh pass has another schedule) and launch shapes must not.
+	for (auto& c : o->gcol) {
+		double sep = -1;
+		if (!rc && o->tune_radix) {
+			o->no_col = true;
+			if (!(rc = build_tables(o, &c.g.meshes))) sep = timed([&] { return middle_all(o, st); });
+			c.g.sh[0].f = 1;
+		}
 		o->no_col = false;
-		std::vector<std::pair<Group*, Group>> keep;
-		for (std::vector<Group>* gs : { &o->gy, &o->gz, &o->gy2, &o->gml, &o->gyz[0], &o->gyz[1] })
-			for (Group& G : *gs) { keep.push_back({ &G, G }); G.sh[0] = G.sh[1] = LaunchShape{}; }
-		rc = build_tables(o);
-		const double plain = rc ? -1 : timed([&] { return middle_all(o, st); });
-		if (plain >= 0 && plain < tuned) { for (auto& k : keep) k.first->us[0] = k.first->us[1] = plain; }   // the whole middle's time
-		else for (auto& k : keep) *k.first = k.second;
+		if (rc || (rc = build_tables(o, &c.g.meshes))) break;
+		const double own = timed([&] { return middle_all(o, st); });
+		c.g.us[0] = own;
+		if (sep >= 0 && (own < 0 || sep < own)) { c.g.sh[0].f = 2; c.g.us[0] = sep; }
 	}
+	// the passes that lost some of their meshes to columns, again with those that are left
+	if (!rc) rc = build_tables(o);
+	if (!rc) tune_middle(true);
 	o->no_col = false;
 	if (!rc) rc = build_tables(o);
 	(void)hipEventDestroy(e0);
@@ -1003,8 +1032,12 @@ extern "C" int bm_batch_mesh_offset(bm_batch_t o, int mesh, long long* cell_offs
 	return BM_OK;
 }
 
+// A column group's name in reports and schedules: "col_2d", "col_ml" (layers) or "col_z<N.z>".
+static std::string col_name(int kind) { return kind == 0 ? "col_ml" : kind == 1 ? "col_2d" : "col_z" + std::to_string(kind); }
+
 // The pass-size group and slot of a pass name ("x_fwd", "x_inv", "y_fwd", "y_inv", "z",
-// "y2d", "ml_mult"; "_pbc" appended for a group along a periodic axis) and size, or nullptr.
+// "y2d", "yzy4", "yzy8", "ml_mult" or a column group's; "_pbc" appended for a group along a
+// periodic axis) and size, or nullptr.
 static Group* find_group(bm_batch_s* o, std::string pass, int size, int& slot)
 {
 	std::vector<Group>* gs = nullptr;
@@ -1019,6 +1052,7 @@ static Group* find_group(bm_batch_s* o, std::string pass, int size, int& slot)
 	else if (pass == "ml_mult") gs = &o->gml;
 	else if (pass == "yzy4") gs = &o->gyz[0];
 	else if (pass == "yzy8") gs = &o->gyz[1];
+	for (auto& c : o->gcol) if (pass == col_name(c.kind) && c.g.size == size && c.g.full == full) return &c.g;
 	if (!gs) return nullptr;
 	for (Group& G : *gs) if (G.size == size && G.full == full) return &G;
 	return nullptr;
@@ -1046,6 +1080,7 @@ extern "C" int bm_batch_autotune_report(bm_batch_t o, char* out, int cap)
 		for (const Group& G : o->gml) add("ml_mult", G, 0);
 		for (const Group& G : o->gyz[0]) add("yzy4", G, 0);
 		for (const Group& G : o->gyz[1]) add("yzy8", G, 0);
+		for (const auto& c : o->gcol) add(col_name(c.kind).c_str(), c.g, 0);
 	}
 	snprintf(out, (size_t)cap, "%s", r.c_str());
 	return BM_OK;
@@ -1059,12 +1094,17 @@ extern "C" int bm_batch_set_schedule(bm_batch_t o, const char* pass, int size, i
 	if (!G) return fail(BM_ERR_ARG, "bm_batch_set_schedule: no such pass and size in this batch");
 	// the fused thin-mesh pass has one schedule per length (radix 0 only)
 	const bool x = pass[0] == 'x', fft = (pass[0] == 'y' || pass[0] == 'z') && std::strncmp(pass, "yzy", 3) != 0;
+	const bool col = std::strncmp(pass, "col", 3) == 0;
 	const bool f_ok = f == 0 || f == 1 || (!G->full && (f == 2 || (f == -2 && x_half_tile_ok(size))));
-	if ((x && !f_ok) || (!x && f != 0) || per_cu < 0 || per_cu > 64 || radix < 0
+	if ((x && !f_ok) || (col && (f < 0 || f > 2 || per_cu != 0)) || (!x && !col && f != 0) || per_cu < 0 || per_cu > 64 || radix < 0
 		|| (fft && !G->full ? radix >= radix_variants(size) : radix != 0))
 		return fail(BM_ERR_ARG, "bm_batch_set_schedule: shape or radix schedule out of range for this pass");
 	G->sh[slot] = LaunchShape{ f, per_cu, radix };
 	G->us[slot] = 0;
+	// a radix schedule asks for the separate pass
+	if (radix)
+		for (auto& c : o->gcol)
+			for (int b : G->meshes) if (c.g.sh[0].f == 1 && std::find(c.g.meshes.begin(), c.g.meshes.end(), b) != c.g.meshes.end()) c.g.sh[0].f = 0;
 	if (o->exec) { (void)hipGraphExecDestroy(o->exec); o->exec = nullptr; }
 	if (o->graph) { (void)hipGraphDestroy(o->graph); o->graph = nullptr; }
 	int rc;
@@ -1099,6 +1139,7 @@ extern "C" int bm_batch_set_pbc(bm_batch_t o, int mesh, int pbc_x, int pbc_y, in
 	}
 	o->pbc[b] = { pbc_x, pbc_y, pbc_z };
 	for (std::vector<Group>* gs : { &o->gx, &o->gy, &o->gz, &o->gy2, &o->gml, &o->gyz[0], &o->gyz[1] }) gs->clear();
+	o->gcol.clear();
 	build_groups(o);
 	if (o->tuned && !o->autotune) o->tuned = false;
 	return build_tables(o);

@@ -319,13 +319,19 @@ int bm_ode_average_m(bm_ode_t o, double* out3, void* stream);
  * factor, workgroups per CU) on the real tables and keep the fastest;
  * BM_BATCH_AUTOTUNE_RADIX (implies BM_BATCH_AUTOTUNE): the y, z and 2D y passes' radix
  * schedules (alternative plans of each FFT length) are timed as well; results then differ
- * from the default schedules by FP32 rounding (launch shapes alone change no bit).
+ * from the default schedules by FP32 rounding (launch shapes alone change no bit).  Meshes whose
+ * y, z or product passes can run as one column kernel form column groups besides: "col_2d",
+ * "col_ml" (layer stacks) or "col_z<N.z>" by N.y.  Their f chooses: 1 the column kernel, 2 the
+ * separate passes, 0 (default) the column kernel unless a y, z or 2D y pass of the mesh is
+ * pinned to another radix schedule.  The two forms round differently, so only radix tuning
+ * chooses between them, group by group.
  * bm_batch_autotune_report writes the choices and times as text lines
  * ("<pass> <size> f=<f> per_cu=<n> radix=<v> <radices> <us> us"); bm_batch_set_schedule
  * pins one pass-size group's choice (e.g. read back from an earlier report), replacing any
  * pending tuning: f (x passes: 0 = default, 1 the base row tile, 2 twice it, -2 half of it
- * where that holds a whole row group: nx 128 to 768; other passes 0), per_cu (0 = default, <= 64),
- * radix (0 = default; y/z/y2d passes only); BM_ERR_ARG for a pass or size the batch lacks.
+ * where that holds a whole row group: nx 128 to 768; column groups as above; other passes 0),
+ * per_cu (0 = default, <= 64; column groups 0), radix (0 = default; y/z/y2d passes only);
+ * BM_ERR_ARG for a pass or size the batch lacks.
  * bm_batch_set_pbc (before the first bm_batch_run): mesh `mesh` becomes periodic as
  * bm_ode_set_pbc makes one mesh (its demag handle rebuilt as bm_demag_create_pbc with these
  * images, exchange wrapping around; not for layer stacks); its passes along periodic axes
