@@ -322,7 +322,7 @@ template <int NY, int KIND, int NZ, bool FULL, bool PACK = false>
 int launch_col_t(const ColArgs& in, int nb, hipStream_t st)
 {
 	// the z form of one mesh with one workgroup per compute unit: columns 0 and N.x / 2 as one
-	if constexpr (KIND == COL_Z && NZ >= 16 && !PACK)
+	if constexpr (KIND == COL_Z && NZ >= 16 && NY % 3 != 0 && !PACK)
 		if (!in.bt && col_packed(col_shape<NY, KIND, NZ>(in.P).lpk, in.NC, in.ncu)) return launch_col_t<NY, KIND, NZ, FULL, true>(in, nb, st);
 	const ColShape s = col_shape<NY, KIND, NZ>(in.P);
 	ColArgs a = in;
@@ -337,11 +337,14 @@ int launch_col_t(const ColArgs& in, int nb, hipStream_t st)
 #define BM_FOR_COL_SIZES(M) M(4) M(6) M(8) M(12) M(16) M(24) M(32) M(48) M(64) M(96) M(128) M(192) M(256) M(384) M(512) M(768) M(1024)
 constexpr size_t kColLds = 150 * 1024;
 
+// the fewest planes of an open N.z (more than a quarter of it) fit LDS
+template <int NY, int NZ> constexpr bool col_z_fits() { return 3 * (NZ / 4 + 1) * lds_len<NY>() * sizeof(C2<float>) <= kColLds; }
+
 // the layers form with 512 (V = 1) or 1024 threads holds P layers; the latter not for N.y = 1024,
 // whose 16 values per thread do not fit its 128 registers (512x512x3 99 us separate, 141 so)
 template <int NY, int V> bool col_items(int P)
 {
-	if (V == 2 && NY >= 1024) return false;
+	if constexpr (V == 2 && NY >= 1024) return false;
 	const ColShape s = col_shape<NY, COL_LAYERS, V>(P);
 	return s.lds <= kColLds && (long long)P * s.lpk * NY <= (long long)kColItems * s.threads;
 }
@@ -372,12 +375,12 @@ int launch_any(int Ny, int kind, bool full, const ColArgs& a, int nb, hipStream_
 	switch (Ny) {
 #define C_(V_) case V_: \
 		if (kind == 0 && col_items<V_, 1>(a.P)) return full ? launch_col_t<V_, COL_LAYERS, 1, true>(a, nb, st) : launch_col_t<V_, COL_LAYERS, 1, false>(a, nb, st); \
-		if (kind == 0) return full ? launch_col_t<V_, COL_LAYERS, 2, true>(a, nb, st) : launch_col_t<V_, COL_LAYERS, 2, false>(a, nb, st); \
+		if constexpr (V_ < 1024) if (kind == 0) return full ? launch_col_t<V_, COL_LAYERS, 2, true>(a, nb, st) : launch_col_t<V_, COL_LAYERS, 2, false>(a, nb, st); \
 		if (kind == 1) return full ? launch_col_t<V_, COL_2D, 1, true>(a, nb, st) : launch_col_t<V_, COL_2D, 1, false>(a, nb, st); \
-		if (kind == 4) return full ? launch_col_t<V_, COL_Z, 4, true>(a, nb, st) : launch_col_t<V_, COL_Z, 4, false>(a, nb, st); \
-		if (kind == 8) return full ? launch_col_t<V_, COL_Z, 8, true>(a, nb, st) : launch_col_t<V_, COL_Z, 8, false>(a, nb, st); \
-		if (kind == 16) return full ? launch_col_t<V_, COL_Z, 16, true>(a, nb, st) : launch_col_t<V_, COL_Z, 16, false>(a, nb, st); \
-		if (kind == 32) return full ? launch_col_t<V_, COL_Z, 32, true>(a, nb, st) : launch_col_t<V_, COL_Z, 32, false>(a, nb, st); \
+		if constexpr (col_z_fits<V_, 4>()) if (kind == 4) return full ? launch_col_t<V_, COL_Z, 4, true>(a, nb, st) : launch_col_t<V_, COL_Z, 4, false>(a, nb, st); \
+		if constexpr (col_z_fits<V_, 8>()) if (kind == 8) return full ? launch_col_t<V_, COL_Z, 8, true>(a, nb, st) : launch_col_t<V_, COL_Z, 8, false>(a, nb, st); \
+		if constexpr (col_z_fits<V_, 16>()) if (kind == 16) return full ? launch_col_t<V_, COL_Z, 16, true>(a, nb, st) : launch_col_t<V_, COL_Z, 16, false>(a, nb, st); \
+		if constexpr (col_z_fits<V_, 32>()) if (kind == 32) return full ? launch_col_t<V_, COL_Z, 32, true>(a, nb, st) : launch_col_t<V_, COL_Z, 32, false>(a, nb, st); \
 		break;
 	BM_FOR_COL_SIZES(C_)
 #undef C_
