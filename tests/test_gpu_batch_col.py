@@ -139,3 +139,19 @@ def test_column_schedules_refused(gpu):
         with pytest.raises(RuntimeError, match="error 1"):
             b.set_schedule(name, size, **kw)
     b.close()
+
+
+def test_one_group_of_unlike_meshes_follows_the_single_runs(gpu):
+    """One (N.y, N.z) group of 257, 129 and 513 columns and 8, 6 and 5 planes against each mesh alone
+    (2e-6 relative L2, the bar of batched against single runs)."""
+    sizes = [(256, 32, 8), (128, 32, 6), (512, 30, 5)]
+    b = batch(sizes=sizes, stacks=[])
+    M0 = b.M.clone()
+    run(b)
+    for q, (n, h, p) in enumerate(b.meshes):
+        s = api.FMSolver(api.BM_EVAL_RK4, n, h, p, M0[int(b.offsets[q]):int(b.offsets[q + 1])].cpu().numpy())
+        s.set_dt(40e-15)
+        s.run_to_iteration(3)
+        assert (s.M - b.mesh(q)).double().norm() <= 2e-6 * s.M.double().norm()
+        s.close()
+    b.close()

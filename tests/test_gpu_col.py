@@ -135,3 +135,21 @@ def test_2d_lines_of_1024(gpu, n, pbc, col):
     ref = O.OracleDemag(n, H, pbc=pbc)(M0.astype(np.float64))
     assert rel(got, ref) <= 1e-6
     d.close()
+
+
+# the packed form (columns 0 and N.x / 2 as one line): N.z 16 and 32, nx a multiple of 256, one column per
+# workgroup; the shortest and longest lines, ragged ny, the fewest and most planes; periodic y and x
+PACKED = [((256, 8, 6), None), ((256, 16, 5), None), ((256, 30, 8), None), ((256, 60, 7), None), ((512, 128, 5), None), ((256, 250, 8), None),
+          ((256, 512, 5), None), ((1024, 32, 6), None), ((256, 8, 9), None), ((256, 30, 16), None), ((512, 60, 12), None), ((256, 128, 16), None),
+          ((256, 250, 9), None), ((256, 64, 8), (0, 2, 0)), ((512, 128, 16), (0, 2, 0)), ((512, 64, 6), (2, 2, 0)), ((512, 30, 10), (2, 0, 0))]
+
+
+@pytest.mark.parametrize("n,pbc", PACKED, ids=str)
+def test_packed_columns(gpu, n, pbc):
+    if (n[0] // (2 if pbc and pbc[0] else 1)) % torch.cuda.get_device_properties(0).multi_processor_count:
+        pytest.skip("N.x / 2 is not a multiple of the compute units")
+    M0 = api.random_magnetisation(n[0] * n[1] * n[2], 8e5, 7).astype(np.float32)
+    d = api.Demag(n, H, pbc or (0, 0, 0))
+    ref = O.OracleDemag(n, H, Nz_override=nz_open(n[2]), pbc=pbc)(M0.astype(np.float64))
+    assert rel(d.convolute(torch.from_numpy(M0).cuda()).cpu().numpy().astype(np.float64), ref) <= 1e-6
+    d.close()
