@@ -564,9 +564,9 @@ int eval_all(bm_batch_s* o, int step, int par, hipStream_t st)
 // launches after a warm-up, HIP events) on the group's real tables and keep the fastest.
 // Candidates: x passes the default, tile factor {1, 2} x workgroups per CU {1, 2, 4}, and the
 // half-height tile at {2, 4, 8} per CU where the row length has one; y passes {4, 8, 16};
-// z pass {1, 2, 4}; 2D y pass {4, 8, 16}; multilayer product {4, 8, 16}.  Then, with radix tuning, for
-// every column group its meshes' column pass against their separate passes.  Only the FFT passes
-// run (their inputs are recomputed from M by every evaluation), so the state is untouched.
+// z pass {1, 2, 4}; 2D y pass {4, 8, 16}; multilayer product {4, 8, 16}.  Then, with radix tuning,
+// the column pass against the separate passes, per column group.  Only the FFT passes run (their
+// inputs are recomputed from M by every evaluation), so the state is untouched.
 int autotune(bm_batch_s* o, hipStream_t st)
 {
 	hipEvent_t e0 = nullptr, e1 = nullptr;
@@ -653,21 +653,34 @@ int autotune(bm_batch_s* o, hipStream_t st)
 			}
 	};
 	tune_middle(false);
-	// Each column group's time and, with radix tuning, its meshes' column pass against their separate
-	// passes as just tuned.  Without it the forms stay, as they round differently (the compiler's
-	// contractions differ, the thin-mesh pass has another schedule) and launch shapes must not.
-	for (auto& c : o->gcol) {
-		double sep = -1;
-		if (!rc && o->tune_radix) {
-			o->no_col = true;
-			if (!(rc = build_tables(o, &c.g.meshes))) sep = timed([&] { return middle_all(o, st); });
-			c.g.sh[0].f = 1;
+	// The column groups.  Launch shapes must not change a bit and the two forms round differently (the
+	// compiler's contractions differ, the thin-mesh pass has another schedule), so only radix
+	// tuning compares them, by the time of the whole middle: column groups run side by side ahead of the
+	// chain of separate passes, so a group's time alone does not tell (64 films: 4.91 ms a step with
+	// every group on columns, 5.05 with the form that is faster alone).  From every group on columns
+	// each one is tried on its separate passes, against all of them at once.
+	o->no_col = false;
+	auto whole = [&] {
+		if (!rc) rc = build_tables(o);
+		return rc ? -1.0 : timed([&] { return middle_all(o, st); });
+	};
+	auto choose = [&](int f) { for (auto& c : o->gcol) c.g.sh[0].f = f; };
+	if (!rc && o->tune_radix && !o->gcol.empty()) {
+		choose(2);
+		const double none = whole();
+		choose(1);
+		double best = whole();
+		for (auto& c : o->gcol) {
+			c.g.sh[0].f = 2;
+			const double t = whole();
+			if (t >= 0 && (best < 0 || t < 0.99 * best)) best = t; else c.g.sh[0].f = 1;
 		}
-		o->no_col = false;
+		if (none >= 0 && (best < 0 || none < 0.99 * best)) choose(2);
+	}
+	// each group's own time in the form it has
+	for (auto& c : o->gcol) {
 		if (rc || (rc = build_tables(o, &c.g.meshes))) break;
-		const double own = timed([&] { return middle_all(o, st); });
-		c.g.us[0] = own;
-		if (sep >= 0 && (own < 0 || sep < own)) { c.g.sh[0].f = 2; c.g.us[0] = sep; }
+		c.g.us[0] = timed([&] { return middle_all(o, st); });
 	}
 	// the passes that lost some of their meshes to columns, again with those that are left
 	if (!rc) rc = build_tables(o);
