@@ -656,8 +656,8 @@ int autotune(bm_batch_s* o, hipStream_t st)
 	// The column groups.  Launch shapes must not change a bit and the two forms round differently (the
 	// compiler's contractions differ, the thin-mesh pass has another schedule), so only radix
 	// tuning compares them, by the time of the whole middle: column groups run side by side ahead of the
-	// chain of separate passes, so a group's time alone does not tell (64 films: 4.91 ms a step with
-	// every group on columns, 5.05 with the form that is faster alone).  From every group on columns
+	// chain of separate passes, so a group's time alone does not tell (two RK4 steps of 64 films: 4.91 ms with
+	// every group on columns, 5.05 with the forms that are faster alone).  From every group on columns
 	// each one is tried on its separate passes, against all of them at once.
 	o->no_col = false;
 	auto whole = [&] {
