@@ -656,26 +656,45 @@ int autotune(bm_batch_s* o, hipStream_t st)
 	// The column groups.  Launch shapes must not change a bit and the two forms round differently (the
 	// compiler's contractions differ, the thin-mesh pass has another schedule), so only radix
 	// tuning compares them, by the time of the whole middle: column groups run side by side ahead of the
-	// chain of separate passes, so a group's time alone does not tell (two RK4 steps of 64 films: 4.91 ms with
-	// every group on columns, 5.05 with the forms that are faster alone).  From every group on columns
-	// each one is tried on its separate passes, against all of them at once.
+	// chain of separate passes, so a group's time alone does not tell (two RK4 steps of 64 films with the
+	// forms that are faster alone 5.05 ms, with every group on columns 4.91).  From every group on
+	// columns each one is tried on its separate passes, then all of them at once (64 films of bench.py,
+	// RK4 step 2.81 -> 2.77 ms).
 	o->no_col = false;
-	auto whole = [&] {
-		if (!rc) rc = build_tables(o);
-		return rc ? -1.0 : timed([&] { return middle_all(o, st); });
+	// the whole middle as a step runs it, captured where steps are (launched one by one its passes took
+	// 380 to 450 us, in a process's first batch the longest, and 397 captured)
+	auto middle_time = [&]() -> double {
+		if (!o->use_graph) return timed([&] { return middle_all(o, st); });
+		hipGraph_t g = nullptr;
+		hipGraphExec_t ex = nullptr;
+		double t = -1;
+		if (hipStreamBeginCapture(o->gs, hipStreamCaptureModeThreadLocal) != hipSuccess) return -1;
+		const int mrc = middle_all(o, o->gs);
+		if (hipStreamEndCapture(o->gs, &g) == hipSuccess && !mrc && hipGraphInstantiate(&ex, g, nullptr, nullptr, 0) == hipSuccess)
+			t = timed([&] { return hipGraphLaunch(ex, st) == hipSuccess ? (int)BM_OK : (int)BM_ERR_HIP; });
+		if (ex) (void)hipGraphExecDestroy(ex);
+		if (g) (void)hipGraphDestroy(g);
+		return t;
 	};
-	auto choose = [&](int f) { for (auto& c : o->gcol) c.g.sh[0].f = f; };
-	if (!rc && o->tune_radix && !o->gcol.empty()) {
-		choose(2);
-		const double none = whole();
-		choose(1);
-		double best = whole();
-		for (auto& c : o->gcol) {
-			c.g.sh[0].f = 2;
-			const double t = whole();
-			if (t >= 0 && (best < 0 || t < 0.99 * best)) best = t; else c.g.sh[0].f = 1;
+	// The choice that a sets against the one that b sets, in turn (the clocks may still be rising):
+	// whether b is the faster by a percent or more.
+	auto faster = [&](auto a, auto b) {
+		double t[2] = { 1e30, 1e30 };
+		for (int r = 0; r < 6 && !rc; r++) {
+			if (r & 1) b(); else a();
+			if ((rc = build_tables(o))) break;
+			const double u = middle_time();
+			if (u >= 0) t[r & 1] = std::min(t[r & 1], u);
 		}
-		if (none >= 0 && (best < 0 || none < 0.99 * best)) choose(2);
+		return t[1] < 0.99 * t[0];
+	};
+	if (o->tune_radix && !o->gcol.empty()) {
+		for (auto& c : o->gcol) c.g.sh[0].f = 1;
+		for (auto& c : o->gcol) c.g.sh[0].f = faster([&] { c.g.sh[0].f = 1; }, [&] { c.g.sh[0].f = 2; }) ? 2 : 1;
+		std::vector<int> f;
+		for (auto& c : o->gcol) f.push_back(c.g.sh[0].f);
+		auto set = [&](bool none) { for (size_t q = 0; q < f.size(); q++) o->gcol[q].g.sh[0].f = none ? 2 : f[q]; };
+		set(faster([&] { set(false); }, [&] { set(true); }));
 	}
 	// each group's own time in the form it has
 	for (auto& c : o->gcol) {
