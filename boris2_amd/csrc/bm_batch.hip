@@ -548,14 +548,21 @@ int middle_all(bm_batch_s* o, hipStream_t st)
 	return rc;
 }
 
-// One field evaluation + stage `step` for every mesh; input magnetisation M (parity 0) or Mb.
-int eval_all(bm_batch_s* o, int step, int par, hipStream_t st)
+// The demag field of every mesh (planar); input magnetisation M (parity 0) or Mb.
+int conv_all(bm_batch_s* o, int par, hipStream_t st)
 {
 	int rc = fan(o, o->gx.size(), st, [&](size_t g, hipStream_t s) {
 		return batch_fwd_x(o->gx[g].size, o->gx[g].full, o->gx[g].sh[0], o->fwd[par][g].h.data(), o->fwd[par][g].d, (int)o->fwd[par][g].h.size(), o->ncu, s); });
 	if (!rc) rc = middle_all(o, st);
 	if (!rc) rc = fan(o, o->gx.size(), st, [&](size_t g, hipStream_t s) {
 		return batch_inv_x_planar(o->gx[g].size, o->gx[g].full, o->gx[g].sh[1], o->inv[g].h.data(), o->inv[g].d, (int)o->inv[g].h.size(), o->ncu, s); });
+	return rc;
+}
+
+// One field evaluation + stage `step` for every mesh.
+int eval_all(bm_batch_s* o, int step, int par, hipStream_t st)
+{
+	int rc = conv_all(o, par, st);
 	if (!rc) rc = batch_stage(o->mcode, step, o->stage[par].d, o->nb, o->choff.d, o->choff.h.back(), st);
 	return rc;
 }
@@ -573,15 +580,15 @@ int autotune(bm_batch_s* o, hipStream_t st)
 	BM_HIP(hipEventCreate(&e0));
 	BM_HIP(hipEventCreate(&e1));
 	int rc = BM_OK;
-	auto timed = [&](auto launch) -> double {
+	auto timed = [&](auto launch, int n = 5) -> double {
 		if (launch() != BM_OK) return -1;
 		(void)hipEventRecord(e0, st);
-		for (int r = 0; r < 5; r++) if (launch() != BM_OK) return -1;
+		for (int r = 0; r < n; r++) if (launch() != BM_OK) return -1;
 		(void)hipEventRecord(e1, st);
 		if (hipEventSynchronize(e1) != hipSuccess) return -1;
 		float ms = 0;
 		(void)hipEventElapsedTime(&ms, e0, e1);
-		return 1e3 * ms / 5;
+		return 1e3 * ms / n;
 	};
 	auto pick = [&](Group& G, int slot, const std::vector<LaunchShape>& cands, bool retable, auto launch) {
 		double bt = 1e30;
@@ -655,38 +662,37 @@ int autotune(bm_batch_s* o, hipStream_t st)
 	tune_middle(false);
 	// The column groups.  Launch shapes must not change a bit and the two forms round differently (the
 	// compiler's contractions differ, the thin-mesh pass has another schedule), so only radix
-	// tuning compares them, by the time of the whole middle: column groups run side by side ahead of the
-	// chain of separate passes, so a group's time alone does not tell (two RK4 steps of 64 films with the
-	// forms that are faster alone 5.05 ms, with every group on columns 4.91).  From every group on
-	// columns each one is tried on its separate passes, then all of them at once (64 films of bench.py,
-	// RK4 step 2.81 -> 2.77 ms).
+	// tuning compares them, by the time of four convolutions of all meshes as a step runs them,
+	// captured where steps are.  Less does not tell: column groups run side by side ahead of the chain
+	// of separate passes, which every mesh waits for (RK4 step of bench.py's 64 films 2.81 ms with every
+	// group on columns, 2.91 as chosen by the middle launched pass by pass, 2.76 so; of 8 films 0.40 ms,
+	// 0.51 as chosen by the middle captured alone, 0.37 to 0.41 so).
 	o->no_col = false;
-	// the whole middle as a step runs it, captured where steps are (launched one by one its passes took
-	// 380 to 450 us, in a process's first batch the longest, and 397 captured)
-	auto middle_time = [&]() -> double {
-		if (!o->use_graph) return timed([&] { return middle_all(o, st); });
+	auto convs = [&](hipStream_t s) { int r = BM_OK; for (int q = 0; q < 4 && !r; q++) r = conv_all(o, 0, s); return r; };
+	auto conv_time = [&]() -> double {
+		if (!o->use_graph) return timed([&] { return convs(st); }, 2);
 		hipGraph_t g = nullptr;
 		hipGraphExec_t ex = nullptr;
 		double t = -1;
 		if (hipStreamBeginCapture(o->gs, hipStreamCaptureModeThreadLocal) != hipSuccess) return -1;
-		const int mrc = middle_all(o, o->gs);
-		if (hipStreamEndCapture(o->gs, &g) == hipSuccess && !mrc && hipGraphInstantiate(&ex, g, nullptr, nullptr, 0) == hipSuccess)
-			t = timed([&] { return hipGraphLaunch(ex, st) == hipSuccess ? (int)BM_OK : (int)BM_ERR_HIP; });
+		const int crc = convs(o->gs);
+		if (hipStreamEndCapture(o->gs, &g) == hipSuccess && !crc && hipGraphInstantiate(&ex, g, nullptr, nullptr, 0) == hipSuccess)
+			t = timed([&] { return hipGraphLaunch(ex, st) == hipSuccess ? (int)BM_OK : (int)BM_ERR_HIP; }, 2);
 		if (ex) (void)hipGraphExecDestroy(ex);
 		if (g) (void)hipGraphDestroy(g);
 		return t;
 	};
 	// The choice that a sets against the one that b sets, in turn (the clocks may still be rising):
-	// whether b is the faster by a percent or more.
+	// whether b is the faster by two percent or more (repeats differ by up to one).
 	auto faster = [&](auto a, auto b) {
 		double t[2] = { 1e30, 1e30 };
-		for (int r = 0; r < 6 && !rc; r++) {
+		for (int r = 0; r < 4 && !rc; r++) {
 			if (r & 1) b(); else a();
 			if ((rc = build_tables(o))) break;
-			const double u = middle_time();
+			const double u = conv_time();
 			if (u >= 0) t[r & 1] = std::min(t[r & 1], u);
 		}
-		return t[1] < 0.99 * t[0];
+		return t[1] < 0.98 * t[0];
 	};
 	if (o->tune_radix && !o->gcol.empty()) {
 		for (auto& c : o->gcol) c.g.sh[0].f = 1;
