@@ -16,7 +16,7 @@ SIZES = [(64, 96, 1), (256, 64, 1), (64, 48, 2), (128, 32, 4), (256, 32, 8), (25
 STACKS = [(64, 48, 3), (96, 32, 7), (32, 64, 12)]
 
 
-def batch(autotune=False, sizes=SIZES, stacks=STACKS, pbc=None):
+def batch(autotune=False, sizes=SIZES, stacks=STACKS, use_graph=True):
     rng = np.random.default_rng(31)
     meshes, M0, layers = [], [], []
     for q, n in enumerate(list(sizes) + list(stacks)):
@@ -25,7 +25,7 @@ def batch(autotune=False, sizes=SIZES, stacks=STACKS, pbc=None):
         M0.append(api.random_magnetisation(n[0] * n[1] * n[2], p.Ms, 80 + q).astype(np.float32))
         hz = [4e-9 if l % 2 else 8e-9 for l in range(n[2])]
         layers.append(dict(hz=hz, z0=[12e-9 * l for l in range(n[2])]) if q >= len(sizes) else None)
-    return api.BatchSolver(api.BM_EVAL_RK4, meshes, M0, layers=layers, autotune=autotune, pbc=pbc)
+    return api.BatchSolver(api.BM_EVAL_RK4, meshes, M0, layers=layers, autotune=autotune, use_graph=use_graph)
 
 
 def run(b, steps=3):
@@ -106,10 +106,11 @@ def test_plain_tuning_changes_no_bit_and_its_report_applies(gpu):
         s.close()
 
 
-def test_radix_tuning_chooses_per_group(gpu):
+@pytest.mark.parametrize("use_graph", [True, False])
+def test_radix_tuning_chooses_per_group(gpu, use_graph):
     """Radix tuning may take either form of any group; its report, applied to another batch, runs the
     same forms."""
-    a, t = batch(), batch(autotune="radix")
+    a, t = batch(), batch(autotune="radix", use_graph=use_graph)
     want, got = run(a), run(t)
     assert (want - got).double().norm() <= 1e-6 * want.double().norm()
     rep = t.autotune_report()

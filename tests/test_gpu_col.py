@@ -70,6 +70,7 @@ def test_layers(gpu, nx, ny, L, pbc):
     d.close()
 
 
+# of these only (512, 128, 12) packs the two columns (N.z 16 or 32, 2^a N.y); test_packed_columns has the form
 @pytest.mark.parametrize("n", [(256, 64, 1), (256, 33, 8), (256, 24, 3), (512, 32, 2), (512, 128, 12), (256, 96, 6), (512, 100, 1)])
 def test_first_and_last_column_as_one(gpu, n):
     """N.x / 2 a multiple of the compute units: columns 0 and N.x / 2 share a workgroup."""
@@ -80,6 +81,7 @@ def test_first_and_last_column_as_one(gpu, n):
     d.close()
 
 
+# layers never pack: one column more than the compute units
 @pytest.mark.parametrize("nx,ny,L", [(256, 32, 3), (256, 64, 6), (512, 24, 4)])
 def test_layers_first_and_last_column_as_one(gpu, nx, ny, L):
     z0 = [8e-9 * l for l in range(L)]

@@ -1,6 +1,6 @@
 """GPU tests of the fused thin-mesh pass (the y, z, y passes of a mesh with N.z = 4 or 8 and a
-power-of-two N.y as one kernel that never writes the full spectra; by default from 512 x 512
-cells per plane, here forced at every size with BM_YZY=2): the demag field against the FP64
+power-of-two N.y as one kernel that never writes the full spectra; by default for N.z = 4 from
+N.y = 1024, here forced at every size with BM_YZY=2): the demag field against the FP64
 oracle and against the separate passes (BM_YZY=0), the add and energy output modes, an
 RKDP54 thin-film trajectory against the oracle, and batches whose thin meshes take it."""
 import numpy as np
@@ -20,7 +20,7 @@ def rel_l2(a, b):
 
 
 def demag(n, monkeypatch, fused):
-    # 2: the fused pass at any size (by default it starts at 512 x 512 cells per plane)
+    # 2: the fused pass at any size (by default N.z = 4 from N.y = 1024)
     monkeypatch.setenv("BM_YZY", "2" if fused else "0")
     return api.Demag(n, H)
 
