@@ -5,6 +5,7 @@ import numpy as np
 import pytest
 import torch
 
+import oracle_lib as O
 from boris2_amd import api
 from test_gpu_adjoint import oracle_grads, problem
 
@@ -23,6 +24,26 @@ def test_adjoint_rows_match_oracle(gpu, n):
     eg, ea = np.linalg.norm(g - g0) / np.linalg.norm(g0), abs(ga - ga0) / abs(ga0)
     print(f"{n}: loss {abs(L - L0):.2e}, dL/dMs rel L2 {eg:.2e}, dL/damp rel {ea:.2e}")
     # the bounds of the 40-step comparison of the same problem (FP32 forward's departure, linear in the steps)
+    assert abs(L - L0) <= 1e-6
+    assert eg <= 5e-5
+    assert ea <= 5e-5
+    r.close()
+
+
+@pytest.mark.parametrize("n,pbc", [((32, 16, 1), (0, 2, 0)), ((64, 12, 4), (0, 2, 2)), ((16, 6, 4), (0, 0, 1))], ids=str)
+def test_adjoint_rows_with_periodic_y_and_z(gpu, n, pbc):
+    """Open x keeps the row kernels, whose exchange then wraps around along the other axes."""
+    n, p, Ms, m0, mt = problem(n, seed=sum(n))
+    dt, steps = 250e-15, 8
+    a = O.OracleAdjoint(n, (4e-9,) * 3, p, Ms, dt, steps, pbc=pbc)
+    L0, _ = a.forward(m0, mt)
+    g0, ga0 = a.backward(m0, mt)
+    r = api.RK4Adjoint(n, (4e-9,) * 3, p, torch.tensor(Ms, dtype=torch.float32), dt, steps, 3, pbc=pbc)
+    L, _ = r.forward(torch.tensor(m0, dtype=torch.float32), torch.tensor(mt, dtype=torch.float32))
+    g, ga = r.backward()
+    g = g.cpu().numpy().astype(np.float64)
+    eg, ea = np.linalg.norm(g - g0) / np.linalg.norm(g0), abs(ga - ga0) / abs(ga0)
+    print(f"{n} {pbc}: loss {abs(L - L0):.2e}, dL/dMs rel L2 {eg:.2e}, dL/damp rel {ea:.2e}")
     assert abs(L - L0) <= 1e-6
     assert eg <= 5e-5
     assert ea <= 5e-5
